@@ -641,7 +641,7 @@ static __global__ void k_edge_flux(FieldGeom g, int ld, const double *__restrict
   pn.p00 = P(0, 0); pn.p10 = P(1, 0); pn.p20 = P(2, 0); pn.pm10 = P(-1, 0);
   pn.p0p = P(0, 1); pn.p0m = P(0, -1); pn.p1p = P(1, 1); pn.p1m = P(1, -1);
   R f[4];
-  const Gas<R> gas = gas_of<R>(g.gamma, g.gas);
+  const Gas<R> gas = gas_of<R>(g.gamma, g.gas[0], g.gas[1], g.gas[2]);
   if (g.quad) {  // normal of the right (i-edge) or top (j-edge) edge of cell (i, j)
     const size_t gc = (size_t)(i + g.nh - 1) + (size_t)(j + g.nh - 1) * (size_t)g.quad_ncx;
     const size_t n = (size_t)g.quad_n;

@@ -66,7 +66,7 @@ int BatchEngine::init(int n, const cato_config *cfgs, const cato_geom *geoms, in
   count_off = off;
   off += 256;
   cursor_off = off;
-  off += align256((size_t)nstages * kNumXcd * sizeof(int));
+  off += align256((size_t)nstages * kCursorInts * sizeof(int));
   pass_off = off;
   off += align256((size_t)(nstages + 1) * pin.size() * sizeof(PressurePass));
   total_bytes = off;
@@ -104,7 +104,7 @@ int BatchEngine::init(int n, const cato_config *cfgs, const cato_geom *geoms, in
                      stream));
   BCK(hipMemcpyAsync(mem + refs_off, refs.data(), n * sizeof(BatchSolveRef), hipMemcpyHostToDevice, stream));
   BCK(hipMemcpyAsync(mem + count_off, &nitems, sizeof(int), hipMemcpyHostToDevice, stream));
-  BCK(hipMemsetAsync(mem + cursor_off, 0, (size_t)nstages * kNumXcd * sizeof(int), stream));
+  BCK(hipMemsetAsync(mem + cursor_off, 0, (size_t)nstages * kCursorInts * sizeof(int), stream));
   hipDeviceProp_t prop;
   int dev = 0;
   BCK(hipGetDevice(&dev));
@@ -204,13 +204,13 @@ int BatchEngine::launch_step(bool first) {
     b.variant = reinterpret_cast<const int *>(mem + variant_off);
     b.items = reinterpret_cast<const BatchItem *>(mem + items_off);
     b.count = reinterpret_cast<const int *>(mem + count_off);
-    b.cursor = reinterpret_cast<int *>(mem + cursor_off) + (size_t)s * kNumXcd;
+    b.cursor = reinterpret_cast<int *>(mem + cursor_off) + (size_t)s * kCursorInts;
     launcher(dim3((unsigned)grid), stream, b);
     BCK(hipGetLastError());
   }
   hipLaunchKernelGGL(batch_finalize_kernel, dim3((unsigned)n), dim3(kThreads), 0, stream,
                      reinterpret_cast<const BatchSolveRef *>(mem + refs_off), 2, reinterpret_cast<int *>(mem + cursor_off),
-                     nstages * kNumXcd);
+                     nstages * kCursorInts);
   BCK(hipGetLastError());
   return CATO_OK;
 }
@@ -253,7 +253,7 @@ int BatchEngine::run(const double *max_time, const double *contour_dt, long long
     L[k].max_iterations = max_iterations;
   }
   BCK(hipMemcpyAsync(mem + loops_off, L.data(), n * sizeof(LoopState), hipMemcpyHostToDevice, stream));
-  BCK(hipMemsetAsync(mem + cursor_off, 0, (size_t)nstages * kNumXcd * sizeof(int), stream));  // outside any graph
+  BCK(hipMemsetAsync(mem + cursor_off, 0, (size_t)nstages * kCursorInts * sizeof(int), stream));  // outside any graph
   int rc = upload_args();  // synchronises, so L may go
   if (rc) return rc;
   if ((rc = compact(L))) return rc;  // every solve live again (a batch may be run more than once)

@@ -440,8 +440,8 @@ __host__ __device__ inline void gas_constants(double gamma, double out[3]) {
   out[1] = 2.0 * ((gamma - 1.0) / (gamma + 1.0));
   out[2] = (gamma + 1.0) / (2.0 * gamma);
 }
-template <typename R> __device__ inline Gas<R> gas_of(double gamma, const double gc[3]) {
-  return Gas<R>{R(gamma), R(gc[0]), R(gc[1]), R(gc[2])};
+template <typename R> __device__ inline Gas<R> gas_of(double gamma, double gg, double cr2, double hf) {
+  return Gas<R>{R(gamma), R(gg), R(cr2), R(hf)};
 }
 
 // SLAU family: slau_solver.fypp:355-490.  With D = FastOps: every numerator is

@@ -144,13 +144,13 @@ int server_tables(cato_server *S) {
   S->count_off = off;
   off += 256;
   S->cursor_off = off;
-  off += a((size_t)S->nstages * kNumXcd * sizeof(int));
+  off += a((size_t)S->nstages * kCursorInts * sizeof(int));
   S->pass_off = off;
   off += a((size_t)(S->nstages + 1) * n * sizeof(PressurePass));
   S->table_bytes = off;
   int rc = hip_check(hipMalloc(&S->table_mem, S->table_bytes), "server tables");
   if (rc) return rc;
-  return hip_check(hipMemset(S->table_mem + S->cursor_off, 0, (size_t)S->nstages * kNumXcd * sizeof(int)),
+  return hip_check(hipMemset(S->table_mem + S->cursor_off, 0, (size_t)S->nstages * kCursorInts * sizeof(int)),
                    "server cursors");
 }
 
@@ -368,7 +368,7 @@ int enqueue_tick(cato_server *S, bool first_fresh, int grid, int resident) {
         b.variant = reinterpret_cast<const int *>(S->table_mem + S->variant_off);
         b.items = reinterpret_cast<const BatchItem *>(S->table_mem + S->items_off);
         b.count = reinterpret_cast<const int *>(S->table_mem + S->count_off);
-        b.cursor = reinterpret_cast<int *>(S->table_mem + S->cursor_off) + (size_t)s * kNumXcd;
+        b.cursor = reinterpret_cast<int *>(S->table_mem + S->cursor_off) + (size_t)s * kCursorInts;
         S->launcher(dim3((unsigned)grid), S->stream, b);
       }
       for (int k : S->big) {
@@ -384,7 +384,7 @@ int enqueue_tick(cato_server *S, bool first_fresh, int grid, int resident) {
     }
     hipLaunchKernelGGL(batch_finalize_kernel, dim3((unsigned)resident), dim3(kThreads), 0, S->stream,
                        reinterpret_cast<const BatchSolveRef *>(S->table_mem + S->refs_off), 2,
-                       reinterpret_cast<int *>(S->table_mem + S->cursor_off), S->nstages * kNumXcd);
+                       reinterpret_cast<int *>(S->table_mem + S->cursor_off), S->nstages * kCursorInts);
   }
   return hip_check(hipGetLastError(), "server step");
 }
@@ -519,7 +519,7 @@ int cato_server_tick(cato_server *S, int *n_resident, int *n_queued, int *n_comp
     drop_tick_graph(S);
     if ((rc = server_upload(S, S->nitems, S->ids))) return rc;
     // work cursors start at zero (the finalize kernel resets them after every step)
-    if ((rc = hip_check(hipMemsetAsync(S->table_mem + S->cursor_off, 0, (size_t)S->nstages * kNumXcd * sizeof(int),
+    if ((rc = hip_check(hipMemsetAsync(S->table_mem + S->cursor_off, 0, (size_t)S->nstages * kCursorInts * sizeof(int),
                                        S->stream), "cursors")))
       return rc;
     S->dirty = false;

@@ -103,16 +103,26 @@ __device__ inline int wave_or(int v) {
 }
 
 // The four variables of a strided set at one cell.
-__device__ inline Prim<double> load4(const double *p, size_t off, long long fstride) {
+// Stage arguments as the tile code takes them: a kernel's own argument, or an
+// entry of the batched kernel's table read through the constant address space
+// (batch_kernel.hpp), so every function below is generic in their type.  The
+// arrays they point at are device memory: a pointer that comes out of a table is
+// generic to the compiler, which would then use flat accesses, so each is marked
+// global where it is used.
+template <typename T> using GlobalPtr = __attribute__((address_space(1))) T *;
+template <typename T> __device__ inline GlobalPtr<T> global(T *p) { return (GlobalPtr<T>)p; }
+
+__device__ inline Prim<double> load4(const double *set, size_t off, long long fstride) {
   const size_t fs = (size_t)fstride;
   return Prim<double>{p[off], p[off + fs], p[off + 2 * fs], p[off + 3 * fs]};
+  auto p = global(set);
 }
 
 // Sub-domain of a split solve: halo'd cell (gi, gj) when a side takes its
 // ghosts from the halo store.  The physical sides map first (as the reference
 // fills boundary ghosts after the exchange, over the full transverse extent),
 // then the cell is interior, in an exchanged strip or in an exchanged corner.
-__device__ inline Prim<double> load_prim_split(const StageArgs &a, int gi, int gj) {
+template <class Args> __device__ inline Prim<double> load_prim_split(Args &a, int gi, int gj) {
   const int ni = a.ni, nj = a.nj, nh = a.nh;
   const bool xh = (gi > ni && (a.halo_mask & 1)) || (gi < 1 && (a.halo_mask & 2));
   const bool yh = (gj > nj && (a.halo_mask & 4)) || (gj < 1 && (a.halo_mask & 8));
@@ -143,7 +153,7 @@ __device__ inline Prim<double> load_prim_split(const StageArgs &a, int gi, int g
       pos = (size_t)ky * len + (size_t)kx;
     }
     stride = (size_t)nh * len;
-    const double *h = a.halo + halo_region_offset(region, ni, nj, nh) + pos;
+    auto h = global(a.halo) + halo_region_offset(region, ni, nj, nh) + pos;
     pr = Prim<double>{h[0], h[stride], h[2 * stride], h[3 * stride]};
   }
   if (fu) pr.u = -pr.u;
@@ -155,7 +165,7 @@ __device__ inline Prim<double> load_prim_split(const StageArgs &a, int gi, int g
 // primitives of a state are those fluid_t%calculate_derived_quantities gives
 // for it (written by the stage that produced the state), or the caller's on
 // the first stage after cato_set_primitive.
-__device__ inline Prim<double> load_prim(const StageArgs &a, int gi, int gj) {
+template <class Args> __device__ inline Prim<double> load_prim(Args &a, int gi, int gj) {
   if (a.halo_mask) return load_prim_split(a, gi, gj);
   bool fu, fv;
   int si = map_axis(gi, a.ni, a.bc[0], a.bc[1], fu);
@@ -181,14 +191,14 @@ __device__ inline Prim<double> load_prim(const StageArgs &a, int gi, int gj) {
 // neighbouring tiles re-read (1.5% faster there; the precision form, which
 // re-reads its input state at the cell, is better off without the hints).
 template <bool NT> __device__ inline double ld_cell(const double *p) {
-  if constexpr (NT) return __builtin_nontemporal_load(p);
-  return *p;
+  if constexpr (NT) return __builtin_nontemporal_load(global(p));
+  return *global(p);
 }
 template <bool NT> __device__ inline void st_cell(double *p, double x) {
   if constexpr (NT) {
-    __builtin_nontemporal_store(x, p);
+    __builtin_nontemporal_store(x, global(p));
   } else {
-    *p = x;
+    *global(p) = x;
   }
 }
 
@@ -197,7 +207,7 @@ template <bool NT> __device__ inline void st_cell(double *p, double x) {
 // form's previous stage would have stored), BC mapping and the +x outflow
 // fill included.  The form stores no primitive arrays: 64 B/cell less HBM
 // traffic per stage for the price of the recovery on halo cells.
-__device__ inline Prim<double> load_recovered(const StageArgs &a, int gi, int gj) {
+template <class Args> __device__ inline Prim<double> load_recovered(Args &a, int gi, int gj) {
   bool fu, fv;
   // the pressure input's ghosts need the whole column (its largest pressure):
   // a pass before the stage stores them in column ni+1 of the primitive arrays
@@ -209,9 +219,8 @@ __device__ inline Prim<double> load_recovered(const StageArgs &a, int gi, int gj
   int sj = map_axis(gj, a.nj, a.bc[2], a.bc[3], fv);
   size_t off = (size_t)(sj - 1) * a.pitch + (size_t)(si - 1);
   double cs;
-  const size_t fs = (size_t)a.fstride;
-  Prim<double> pr = cons_to_prim_fast(a.uk[0][off], a.uk[0][off + fs], a.uk[0][off + 2 * fs],
-                                      a.uk[0][off + 3 * fs], a.gamma, a.gamma - 1.0, 0, &cs);
+  const Prim<double> U = load4(a.uk[0], off, a.fstride);
+  Prim<double> pr = cons_to_prim_fast(U.rho, U.u, U.v, U.p, a.gamma, a.gamma - 1.0, 0, &cs);
   if (fu) pr.u = -pr.u;
   if (fv) pr.v = -pr.v;
   if (gi > a.ni && a.bc[0] == BC_OUTFLOW) pr = outflow_ghost(pr, a.gamma, a.bc_pressure);
@@ -306,8 +315,9 @@ using RedSmem = RedSmemT<kThreads / 64>;
 // (IeeeOps, or FastOps on in-range tiles).  GEOM: general quadrilateral cells,
 // the normal read from the per-cell geometry (the right edge of its left cell
 // for an i-edge, the top edge for a j-edge).
-template <int FLUX, int LIMC, typename R, int TX, int TY, class D, class DF, bool GEOM, int KIND, int NT, bool SPLIT>
-__device__ __forceinline__ bool tile_edge(const StageArgs &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm, int i0, int j0,
+template <int FLUX, int LIMC, typename R, int TX, int TY, class D, class DF, bool GEOM, int KIND, int NT, bool SPLIT,
+          class Args>
+__device__ __forceinline__ bool tile_edge(Args &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm, int i0, int j0,
                                           bool idir, int ex, int ey, R (&f)[4]) {
   constexpr int H = halo_of<LIMC>();
   constexpr int RX = TX + 2 * H;
@@ -351,13 +361,13 @@ __device__ __forceinline__ bool tile_edge(const StageArgs &a, TileSmem<LIMC, R, 
   if constexpr (GEOM) {
     const size_t gc = (size_t)(ci + a.nh - 1) + (size_t)(cj + a.nh - 1) * (size_t)a.quad_ncx;
     const size_t n = (size_t)a.quad_n;
-    s.nx = (R)a.quad[(idir ? Q_NRX : Q_NTX) * n + gc];
-    s.ny = (R)a.quad[(idir ? Q_NRY : Q_NTY) * n + gc];
+    s.nx = (R)global(a.quad)[(idir ? Q_NRX : Q_NTX) * n + gc];
+    s.ny = (R)global(a.quad)[(idir ? Q_NRY : Q_NTY) * n + gc];
   } else {
     s.nx = idir ? R(1) : R(0);
     s.ny = idir ? R(0) : R(1);
   }
-  edge_flux<R, FLUX, DIR, DF>(gas_of<R>(a.gamma, a.gas), a.low_mach_fix, s, pn, f, &sb);
+  edge_flux<R, FLUX, DIR, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2]), a.low_mach_fix, s, pn, f, &sb);
   return true;
 }
 
@@ -369,8 +379,8 @@ __device__ __forceinline__ bool tile_edge(const StageArgs &a, TileSmem<LIMC, R, 
 // to sfj; the first and last rounds take a single edge direction, folded at
 // compile time.  Otherwise the edges in order, i-edges first, with the
 // direction at run time.
-template <int FLUX, int LIMC, typename R, int TX, int TY, class D, class DF, bool GEOM, int NT, bool SPLIT>
-__device__ inline void edge_pass(const StageArgs &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm, int i0, int j0,
+template <int FLUX, int LIMC, typename R, int TX, int TY, class D, class DF, bool GEOM, int NT, bool SPLIT, class Args>
+__device__ inline void edge_pass(Args &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm, int i0, int j0,
                                  R (&hold)[4]) {
   constexpr int NIE = (TX + 1) * TY, NJE = TX * (TY + 1);
   const int tid = threadIdx.x;
@@ -434,8 +444,8 @@ __device__ inline void edge_pass(const StageArgs &a, TileSmem<LIMC, R, TX, TY, N
 // kernel); the single-solve launch leaves that to k_outflow_column, since the
 // extra epilogue slows every tile of the fused kernel by ~5%.
 template <int FLUX, int LIMC, typename R, int TX, int TY, bool OUTFLOW_COL = false, bool GEOM = false,
-          int NT = kThreads, bool SPLIT = false>
-__device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm,
+          int NT = kThreads, bool SPLIT = false, class Args>
+__device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm,
                                   RedSmemT<NT / 64> &red) {
   constexpr int H = halo_of<LIMC>();
   constexpr int RX = TX + 2 * H, RY = TY + 2 * H;
@@ -470,15 +480,14 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
   if (inner) {
     const bool check = recover || a.check_input;
     const size_t base = (size_t)(j0 - H - 1) * a.pitch + (size_t)(i0 - H - 1);
-    const size_t fs = (size_t)a.fstride;
     for (int idx = tid; idx < RX * RY; idx += NT) {
       int ly = idx / RX, lx = idx - ly * RX;
       const size_t off = base + (size_t)ly * a.pitch + (size_t)lx;
       Prim<double> pr;
       if (recover) {
         double cs;
-        pr = cons_to_prim_fast(a.uk[0][off], a.uk[0][off + fs], a.uk[0][off + 2 * fs], a.uk[0][off + 3 * fs],
-                               a.gamma, a.gamma - 1.0, 0, &cs);
+        const Prim<double> U = load4(a.uk[0], off, a.fstride);
+        pr = cons_to_prim_fast(U.rho, U.u, U.v, U.p, a.gamma, a.gamma - 1.0, 0, &cs);
       } else {
         pr = load4(a.prim[0], off, a.fstride);
       }
@@ -568,17 +577,17 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
         // quad_cell geometry of the cell: min_dx / min_dy, bottom / right / top / left lengths, volume
         const size_t gc = (size_t)(gi + nh - 1) + (size_t)(gj + nh - 1) * (size_t)a.quad_ncx;
         const size_t n = (size_t)a.quad_n;
-        dxv = a.quad[Q_MDX * n + gc];
-        dyv = a.quad[Q_MDY * n + gc];
-        lb = a.quad[Q_LEN0 * n + gc];
-        lr = a.quad[Q_LEN1 * n + gc];
-        lt = a.quad[Q_LEN2 * n + gc];
-        ll = a.quad[Q_LEN3 * n + gc];
-        vol = a.quad[Q_VOL * n + gc];
+        dxv = global(a.quad)[Q_MDX * n + gc];
+        dyv = global(a.quad)[Q_MDY * n + gc];
+        lb = global(a.quad)[Q_LEN0 * n + gc];
+        lr = global(a.quad)[Q_LEN1 * n + gc];
+        lt = global(a.quad)[Q_LEN2 * n + gc];
+        ll = global(a.quad)[Q_LEN3 * n + gc];
+        vol = global(a.quad)[Q_VOL * n + gc];
       } else {
-        dxv = a.dxi[gi + nh - 1];
-        dyv = a.dyj[gj + nh - 1];
-        double l1 = a.lxi[gi + nh - 1], l2 = a.lyj[gj + nh - 1];
+        dxv = global(a.dxi)[gi + nh - 1];
+        dyv = global(a.dyj)[gj + nh - 1];
+        double l1 = global(a.lxi)[gi + nh - 1], l2 = global(a.lyj)[gj + nh - 1];
         // edge-length equalisation (quad_cell.f90:110-112) over (l1, l2, l1, l2)
         double mx = fmax2(l1, l2), mn = fmin2(l1, l2);
         lb = l1, lr = l2, lt = l1, ll = l2;
@@ -597,7 +606,7 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
     double fst[4] = {0.0, 0.0, 0.0, 0.0};  // issued before the flux balance to hide their latency
     if (conv) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) fst[v] = a.conv_first[0][off + v * fs];
+      for (int v = 0; v < 4; ++v) fst[v] = global(a.conv_first[0])[off + v * fs];
     }
     // precision form, rectilinear cells (lr == ll, lt == lb): lengths over the volume
     const double sx = kExact ? 0.0 : lr * inv_vol, sy = kExact ? 0.0 : lb * inv_vol;
@@ -628,7 +637,7 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
           L = -(((Fi - Fim) * sx) + ((Gj - Gjm) * sy));
       }
       // time_derivative's energy source (mod_fluid.f90:500-509): a plain sum
-      if (v == 3 && a.src_E) L = L + a.src_E[off];
+      if (v == 3 && a.src_E) L = L + global(a.src_E)[off];
       // the field operators' sum (its epsilon flush only shapes rounding at 1e-16,
       // which the precision form leaves out as in its flux balance)
       auto sum = [](double x, double y) { return kExact ? op_add(x, y) : x + y; };
@@ -636,11 +645,11 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
       if (a.mode == MODE_RESIDUAL) {
         r = L;
       } else if (a.mode == MODE_FIRST) {
-        r = sum(a.uk[0][off + v * fs], L * (a.c * dt));
+        r = sum(global(a.uk[0])[off + v * fs], L * (a.c * dt));
       } else if (a.mode == MODE_BASE) {
         r = sum(ld_cell<kExact>(&a.u0[0][off + v * fs]), L * (dt * a.c));
       } else {
-        double t = sum(ld_cell<kExact>(&a.u0[0][off + v * fs]) * a.a, a.uk[0][off + v * fs] * a.b);
+        double t = sum(ld_cell<kExact>(&a.u0[0][off + v * fs]) * a.a, global(a.uk[0])[off + v * fs] * a.b);
         r = sum(t, L * (a.c * dt));
       }
       nv[v] = r;
@@ -668,10 +677,10 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
     }
     if (kExact && OUTFLOW_COL && gi == ni && a.bc[0] == BC_OUTFLOW) {
       Prim<double> g = outflow_ghost(q, a.gamma, a.bc_pressure);
-      a.prim_out[0][off + 1] = g.rho;
-      a.prim_out[0][off + fs + 1] = g.u;
-      a.prim_out[0][off + 2 * fs + 1] = g.v;
-      a.prim_out[0][off + 3 * fs + 1] = g.p;
+      global(a.prim_out[0])[off + 1] = g.rho;
+      global(a.prim_out[0])[off + fs + 1] = g.u;
+      global(a.prim_out[0])[off + 2 * fs + 1] = g.v;
+      global(a.prim_out[0])[off + 3 * fs + 1] = g.p;
     }
     if (q.rho != q.rho || q.u != q.u || q.v != q.v || q.p != q.p) err |= 1;
     if (a.last_stage) {
@@ -696,7 +705,7 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
       double t = red.s[0][tid];
 #pragma unroll
       for (int k = 1; k < NT / 64; ++k) t = t + red.s[k][tid];
-      a.block_conv[(size_t)tid * (size_t)(a.tiles_x * a.tiles_y) + tile] = t;
+      global(a.block_conv)[(size_t)tid * (size_t)(a.tiles_x * a.tiles_y) + tile] = t;
     }
   }
 
@@ -717,8 +726,8 @@ __device__ inline void stage_tile(const StageArgs &a, int tile, double dt, TileS
         m = (red_min[k] < m) ? red_min[k] : m;
         e |= red_err[k];
       }
-      if (a.block_min) a.block_min[tile] = m;
-      if (a.block_err && e) a.block_err[tile] |= e;
+      if (a.block_min) global(a.block_min)[tile] = m;
+      if (a.block_err && e) global(a.block_err)[tile] |= e;
     }
   }
 }
