@@ -102,7 +102,6 @@ __device__ inline int wave_or(int v) {
   return v;
 }
 
-// The four variables of a strided set at one cell.
 // Stage arguments as the tile code takes them: a kernel's own argument, or an
 // entry of the batched kernel's table read through the constant address space
 // (batch_kernel.hpp), so every function below is generic in their type.  The
@@ -112,10 +111,11 @@ __device__ inline int wave_or(int v) {
 template <typename T> using GlobalPtr = __attribute__((address_space(1))) T *;
 template <typename T> __device__ inline GlobalPtr<T> global(T *p) { return (GlobalPtr<T>)p; }
 
+// The four variables of a strided set at one cell.
 __device__ inline Prim<double> load4(const double *set, size_t off, long long fstride) {
   const size_t fs = (size_t)fstride;
-  return Prim<double>{p[off], p[off + fs], p[off + 2 * fs], p[off + 3 * fs]};
   auto p = global(set);
+  return Prim<double>{p[off], p[off + fs], p[off + 2 * fs], p[off + 3 * fs]};
 }
 
 // Sub-domain of a split solve: halo'd cell (gi, gj) when a side takes its
