@@ -122,6 +122,15 @@ struct StageArgs {
   int ugeom, ugeom_pow2;
   double ug[8];
   const LoopState *loop;     // dt source and done flag (may be null -> dt_value)
+  // A step that closes the one before it (latency layout only): fold_n > 0 partial minima and sanity flags
+  // of that step's last stage, which the first stage reduces before its own dt; loop_out (the first and the
+  // second stage), the copy of the loop state that the next stage reads.  No stage writes what another
+  // workgroup of its launch reads, so the state alternates between two copies, as the flags do: err_assign,
+  // block_err[tile] is set (to the flags of err_prev[tile], if any, and the tile's own), not added to
+  int fold_n, err_assign;
+  const double *fold_min;
+  const int *fold_err, *err_prev;
+  LoopState *loop_out;
   double dt_value;
   double *block_min;         // per-block CFL minimum (last stage)
   int *block_err;            // per-block sanity flags

@@ -254,14 +254,20 @@ static int validate_config(const cato_config &c) {
   return CATO_OK;
 }
 
-int default_tile(const cato_config &c, int ni, int nj) {
+// The library's choice of tile: the latency layout up to five of its tiles per CU, 32 x 8 above.  Measured
+// with five schemes in both precisions, us per SSP-RK3 step with 32 x 8 tiles / in the latency layout:
+// 64^2 35-51 / 21-25 (FP64) and 26-35 / 15-17 (FP32 flux); 256^2 35-52 / 32-43 and 25-35 / 21-27;
+// 272^2 (1156 tiles) 40-64 / 36-49 and 28-40 / 23-30; FP64 288^2 (1296 tiles) 40-64 / 42-58.
+constexpr int kLatencyTiles = 5 * 256;
+
+static int default_tile(const cato_config &c, int ni, int nj, bool single) {
   if (c.tile >= 0) return c.tile;
-  (void)ni;
-  (void)nj;
-  return 0;  // 32 x 8
+  const TileShape t = kTiles[kLatencyTile];
+  const long long tiles = (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
+  return single && tiles <= kLatencyTiles ? kLatencyTile : 0;
 }
 
-int Solve::init(const cato_config &c, const cato_geom &g, bool allow_quad) {
+int Solve::init(const cato_config &c, const cato_geom &g, bool single) {
   int rc = validate_config(c);
   if (rc) return rc;
   if (g.ni < c.n_ghost_layers || g.nj < c.n_ghost_layers)
@@ -275,11 +281,12 @@ int Solve::init(const cato_config &c, const cato_geom &g, bool allow_quad) {
   pitch = (ni + (ghost_column_bc(c.bc_plus_x) ? 1 : 0) + 15) & ~15;
   rc = build_geometry(ni, nj, nh, g.node_x, g.node_y, geo);
   if (rc) return rc;
-  if (geo.quad && !allow_quad)
+  if (geo.quad && !single)
     return fail(CATO_ERR_UNSUPPORTED,
                 "general quadrilateral grids run as single solves (cato_ctx); this form takes rectilinear grids");
-  // quad cells: the one tile shape their kernels are instantiated for
-  tile = geo.quad ? kQuadTile : default_tile(c, ni, nj);
+  // quad cells: the tile shapes their kernels are instantiated for
+  tile = default_tile(c, ni, nj, single);
+  if (geo.quad && tile != kLatencyTile) tile = kQuadTile;
   tiles_x = (ni + kTiles[tile].tx - 1) / kTiles[tile].tx;
   tiles_y = (nj + kTiles[tile].ty - 1) / kTiles[tile].ty;
   launcher = stage_launcher(c.flux, c.limiter, c.precision, tile, geo.quad ? 1 : 0);
@@ -289,9 +296,16 @@ int Solve::init(const cato_config &c, const cato_geom &g, bool allow_quad) {
 
 size_t Solve::field_elems() const { return (size_t)pitch * nj; }
 
+// Tiles whose partials lie within device_bytes(): the solve's own, except that those of the latency layout
+// lie in its tail and the 32 x 8 tiles it stands for count here.
+size_t Solve::counted_tiles() const {
+  const TileShape t = kTiles[tile == kLatencyTile ? 0 : tile];
+  return (size_t)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
+}
+
 size_t Solve::device_bytes() const {
   size_t f = field_elems();
-  size_t nb = (size_t)tiles_x * tiles_y;
+  size_t nb = counted_tiles();
   size_t geo_n = (size_t)2 * (ni + 2 * nh) + 2 * (nj + 2 * nh);
   return (12 + 12) * f * sizeof(double) + geo_n * sizeof(double) + (size_t)Q_COUNT * quad_elems() * sizeof(double) +
          nb * (sizeof(double) + sizeof(int)) + sizeof(LoopState) + 4 * sizeof(double) + 1024;
@@ -317,13 +331,28 @@ void Solve::bind(char *base) {
   lyj = p; p += nj + 2 * nh;
   quad = geo.quad ? p : nullptr;
   p += (size_t)Q_COUNT * quad_elems();
-  block_min = p; p += (size_t)tiles_x * tiles_y;
+  block_min = p; p += counted_tiles();
   result = p; p += 4;
   char *c = reinterpret_cast<char *>(p);
   c = reinterpret_cast<char *>(((uintptr_t)c + 255) & ~(uintptr_t)255);
   loop = reinterpret_cast<LoopState *>(c);
   c += sizeof(LoopState);
   block_err = reinterpret_cast<int *>(c);
+}
+
+// What a single solve keeps after its device_bytes(): the second copies of the loop state and the sanity
+// flags (StageArgs::fold_n), and the partials of the latency layout's tiles, more than a batched solve's.
+size_t Solve::tail_bytes() const {
+  return 256 + sizeof(LoopState) + (size_t)tiles_x * tiles_y * (sizeof(double) + 2 * sizeof(int));
+}
+
+void Solve::bind_tail(char *base) {
+  const size_t nb = (size_t)tiles_x * tiles_y;
+  base = reinterpret_cast<char *>(((uintptr_t)base + 255) & ~(uintptr_t)255);
+  loop_b = reinterpret_cast<LoopState *>(base);
+  block_min = reinterpret_cast<double *>(base + sizeof(LoopState));
+  block_err = reinterpret_cast<int *>(block_min + nb);
+  block_err_b = block_err + nb;
 }
 
 int Solve::upload_geometry(hipStream_t s) {
@@ -411,6 +440,21 @@ StageArgs Solve::stage_args(int mode, double a, double b, double c, int in_buf, 
   s.quad_n = (long long)quad_elems();
   s.fstride = (long long)field_elems();
   return s;
+}
+
+// A step of a run of steps: its first stage closes the step before it (`prev`, within the run), instead of
+// a reduction between them.  See StageArgs::fold_n for who reads and writes which copy.
+void Solve::chain_step(std::vector<StageArgs> &st, bool prev) const {
+  StageArgs &a = st[0], &b = st[1];
+  a.fold_n = prev ? tiles_x * tiles_y : 0;
+  a.fold_min = block_min;
+  a.fold_err = block_err;
+  a.loop_out = loop_b;
+  a.block_err = block_err_b;
+  a.err_assign = b.err_assign = 1;
+  b.err_prev = block_err_b;
+  b.loop_out = loop;
+  for (size_t m = 1; m < st.size(); ++m) st[m].loop = loop_b;
 }
 
 // Primitive buffer sets read and written by stage m of an ns-stage step.  P[0]
@@ -935,12 +979,13 @@ int cato_ctx_create(const cato_config *cfg, const cato_geom *geom, cato_ctx **ou
     return rc;
   }
   size_t bytes = c->s.device_bytes();
-  if ((rc = hip_check(hipMalloc(&c->mem, bytes), "device allocation"))) {
+  if ((rc = hip_check(hipMalloc(&c->mem, bytes + c->s.tail_bytes()), "device allocation"))) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     return rc;
   }
   c->s.bind(c->mem);
+  c->s.bind_tail(c->mem + bytes);
   if ((rc = c->s.upload_geometry(c->stream)) || (rc = hip_check(hipStreamSynchronize(c->stream), "sync"))) {
     cato_ctx_destroy(c);
     return rc;
@@ -1190,14 +1235,29 @@ int cato_step(cato_ctx *c, double dt, int *error_code) {
   return CATO_OK;
 }
 
-// One step of the device-side loop (stages with the device dt, then the
-// end-of-step reduction and loop update).
-static int enqueue_step(cato_ctx *c) {
+// Whether steps close each other (chain_step): in the latency layout, whose few tiles (kLatencyTiles) every
+// workgroup reduces by itself under its tile's loads, while nothing else reads the loop state between two
+// steps (the +x pressure input does) or forms norms there (the diagnostics do).  The reduction launch this
+// saves took 4.5 us of every step.
+static bool chained(const cato_ctx *c) {
+  const Solve &s = c->s;
+  return s.tile == kLatencyTile && !c->timing && !s.conv_sums && s.cfg.bc_plus_x != BC_PRESSURE_INPUT;
+}
+
+// n steps of the device-side loop: stages with the device dt, then the end-of-step reduction and loop update
+// (of the last step alone where they are chained).
+static int enqueue_run(cato_ctx *c, long long n) {
   Solve &s = c->s;
-  int rc = launch_stages(c, s.step_stages(s.loop, 0.0));
-  if (rc) return rc;
-  s.prims_valid = false;
-  return launch_reduce(c, 2, true);
+  const bool chain = chained(c);
+  int rc;
+  for (long long k = 0; k < n; ++k) {
+    std::vector<StageArgs> st = s.step_stages(s.loop, 0.0);
+    if (chain) s.chain_step(st, k > 0);
+    if ((rc = launch_stages(c, st))) return rc;
+    s.prims_valid = false;
+    if ((!chain || k == n - 1) && (rc = launch_reduce(c, 2, true))) return rc;
+  }
+  return CATO_OK;
 }
 
 // n steps of the device-side loop.  The arguments of every step are the same
@@ -1210,14 +1270,14 @@ static int enqueue_steps(cato_ctx *c, long long n) {
   long long k = 0;
   int rc = CATO_OK;
   if (n > 0 && s.prims_valid) {
-    if ((rc = enqueue_step(c))) return rc;
+    if ((rc = enqueue_run(c, 1))) return rc;
     k = 1;
   }
   if (c->use_graph && !c->timing && n - k >= kGraphSteps) {
     if (!c->steps_exec) {
       hipGraph_t g = nullptr;
       HIPCK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      for (long long q = 0; q < kGraphSteps && !rc; ++q) rc = enqueue_step(c);
+      rc = enqueue_run(c, kGraphSteps);
       hipError_t e = hipStreamEndCapture(c->stream, &g);
       if (rc || e != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
@@ -1232,9 +1292,7 @@ static int enqueue_steps(cato_ctx *c, long long n) {
     }
     for (; n - k >= kGraphSteps; k += kGraphSteps) HIPCK(hipGraphLaunch(c->steps_exec, c->stream));
   }
-  for (; k < n; ++k)
-    if ((rc = enqueue_step(c))) return rc;
-  return CATO_OK;
+  return n > k ? enqueue_run(c, n - k) : CATO_OK;
 }
 
 static int run_impl(cato_ctx *c, double max_time, long long max_iter, double contour_dt, double constant_dt,

@@ -30,7 +30,6 @@ struct Geometry1D {
   double u[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 };
 int build_geometry(int ni, int nj, int nh, const double *nx, const double *ny, Geometry1D &g);
-int default_tile(const cato_config &c, int ni, int nj);
 int validate_stage_args(const StageArgs &s);
 
 // One solve: configuration, geometry and the device arrays it owns.
@@ -50,6 +49,8 @@ struct Solve {
   double *result = nullptr;
   int *block_err = nullptr;
   LoopState *loop = nullptr;
+  LoopState *loop_b = nullptr;  // the second copies that chained steps alternate with (bind_tail)
+  int *block_err_b = nullptr;
   double *src_E = nullptr;  // energy source field (pitched like U; owned by the caller of bind())
   double *pi_tab = nullptr; // pressure input table: n times, pressures, densities (owned by the caller)
   int pi_n = 0;
@@ -64,13 +65,17 @@ struct Solve {
   bool prims_valid = false; // P[0] holds the caller's primitives (not yet checked by a stage)
   bool prims_stale = false; // precision form: stages left P[0] behind U[cur] (they store no primitives)
 
-  // allow_quad: accept a general quadrilateral grid (single solves; the batched,
-  // served and split forms take rectilinear grids only)
-  int init(const cato_config &c, const cato_geom &g, bool allow_quad = false);
+  // single: the solve has launches of its own (cato_ctx), so it may have a general
+  // quadrilateral grid and the latency layout; the batched, served and split forms
+  // take rectilinear grids and the shared tiles only
+  int init(const cato_config &c, const cato_geom &g, bool single = false);
   size_t quad_elems() const { return geo.quad ? (size_t)(ni + 2 * nh) * (nj + 2 * nh) : 0; }
   size_t field_elems() const;
+  size_t counted_tiles() const;
   size_t device_bytes() const;
   void bind(char *base);
+  size_t tail_bytes() const;
+  void bind_tail(char *base);
   int upload_geometry(hipStream_t s);
   FieldGeom fgeom() const;
   StageArgs stage_args(int mode, double a, double b, double c, int in_buf, int u0_buf, int out_buf, int p_in,
@@ -78,6 +83,7 @@ struct Solve {
   // keep_un: the last stage writes a free state buffer and primitive set instead
   // of U^n and P[0] (a step that may be retried from U^n, subcycle_check)
   std::vector<StageArgs> step_stages(const LoopState *lp, double dt_value, bool keep_un = false) const;
+  void chain_step(std::vector<StageArgs> &st, bool prev) const;
   ConvOut conv_out() const { return ConvOut{conv_sums, conv_norms, conv_hist, kHistCap}; }
 };
 

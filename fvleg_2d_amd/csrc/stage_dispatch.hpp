@@ -13,8 +13,10 @@ struct TileShape {
   int tx, ty;
 };
 constexpr int kNumTiles = 4;
-constexpr TileShape kTiles[kNumTiles] = {{32, 8}, {32, 16}, {16, 16}, {64, 8}};
-// the one tile shape instantiated for general quadrilateral cells
+// the last one, the latency layout, is the library's own choice for small grids
+constexpr TileShape kTiles[kNumTiles + 1] = {{32, 8}, {32, 16}, {16, 16}, {64, 8}, {8, 8}};
+constexpr int kLatencyTile = kNumTiles;
+// the tile shape instantiated for general quadrilateral cells, beside kLatencyTile
 constexpr int kQuadTile = 2;
 
 using StageLauncher = void (*)(dim3 grid, hipStream_t stream, const StageArgs &args);

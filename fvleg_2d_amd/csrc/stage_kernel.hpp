@@ -22,6 +22,7 @@
 // normals.
 #pragma once
 
+#include "loop_state.hpp"
 #include "physics.hpp"
 
 
@@ -83,13 +84,35 @@ __device__ inline Prim<double> outflow_ghost(Prim<double> d, double gamma, doubl
   return g;
 }
 
+// The value of another lane of the row of 16, by a data-parallel-primitives move
+// (no LDS access, which is what a shuffle costs).
+template <int CTRL> __device__ inline int dpp_move(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL> __device__ inline double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = dpp_move<CTRL>((int)b), hi = dpp_move<CTRL>((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ inline int lane_value(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ inline double lane_value(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = lane_value((int)b, lane), hi = lane_value((int)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// v of all 64 lanes (all active) combined by an exact, order-free operation: within
+// quads, eights and rows by DPP (quad_perm xor 1, xor 2, row_half_mirror,
+// row_mirror), then the four rows.  Six shuffles through LDS took 1,000 cycles at
+// the end of every last stage's workgroup.
+template <typename T, class Op> __device__ inline T wave_reduce(T v, Op op) {
+  v = op(v, dpp_move<0xB1>(v));
+  v = op(v, dpp_move<0x4E>(v));
+  v = op(v, dpp_move<0x141>(v));
+  v = op(v, dpp_move<0x140>(v));
+  return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48)));
+}
 template <typename T> __device__ inline T wave_min(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    T w = __shfl_xor(v, o, 64);
-    v = (w < v) ? w : v;
-  }
-  return v;
+  return wave_reduce(v, [](T x, T y) { return (y < x) ? y : x; });
 }
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -97,9 +120,7 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 __device__ inline int wave_or(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
-  return v;
+  return wave_reduce(v, [](int x, int y) { return x | y; });
 }
 
 // Stage arguments as the tile code takes them: a kernel's own argument, or an
@@ -305,6 +326,35 @@ template <int NW> struct RedSmemT {
 };
 using RedSmem = RedSmemT<kThreads / 64>;
 
+// Pressures around an edge whose left cell is at pc (sn, st: strides along the
+// edge's normal and across it).
+template <typename R> __device__ inline PressNbr<R> pressure_nbrs(const R *pc, int sn, int st) {
+  PressNbr<R> pn;
+  pn.p00 = pc[0];
+  pn.p10 = pc[sn];
+  pn.p20 = pc[2 * sn];
+  pn.pm10 = pc[-sn];
+  pn.p0p = pc[st];
+  pn.p0m = pc[-st];
+  pn.p1p = pc[sn + st];
+  pn.p1m = pc[sn - st];
+  return pn;
+}
+
+// Unit normal of the edge right of (idir) or above cell (ci, cj).
+template <bool GEOM, typename R, class Args>
+__device__ inline void edge_normal(Args &a, bool idir, int ci, int cj, EdgeState<R> &s) {
+  if constexpr (GEOM) {
+    const size_t gc = (size_t)(ci + a.nh - 1) + (size_t)(cj + a.nh - 1) * (size_t)a.quad_ncx;
+    const size_t n = (size_t)a.quad_n;
+    s.nx = (R)global(a.quad)[(idir ? Q_NRX : Q_NTX) * n + gc];
+    s.ny = (R)global(a.quad)[(idir ? Q_NRY : Q_NTY) * n + gc];
+  } else {
+    s.nx = idir ? R(1) : R(0);
+    s.ny = idir ? R(0) : R(1);
+  }
+}
+
 // Edge (ex, ey) of a tile, an i-edge (idir) or a j-edge: its L/R
 // reconstruction from the LDS primitives and its flux.  i-edge (ex, ey) lies
 // between tile cells (ex - 1, ey) and (ex, ey), j-edge (ex, ey) between
@@ -342,31 +392,13 @@ __device__ __forceinline__ bool tile_edge(Args &a, TileSmem<LIMC, R, TX, TY, NT,
     recon_var<R, LIM_SUPERBEE, D>(&sp[3][ly][lx], sn, st, sb.pL, sb.pR);
   }
   PressNbr<R> pn;
-  if constexpr (needs_pressure_nbrs<FLUX>()) {
-    const R *pc = &sp[3][ly][lx];
-    pn.p00 = pc[0];
-    pn.p10 = pc[sn];
-    pn.p20 = pc[2 * sn];
-    pn.pm10 = pc[-sn];
-    pn.p0p = pc[st];
-    pn.p0m = pc[-st];
-    pn.p1p = pc[sn + st];
-    pn.p1m = pc[sn - st];
-  }
+  if constexpr (needs_pressure_nbrs<FLUX>()) pn = pressure_nbrs(&sp[3][ly][lx], sn, st);
   // direction code: 0 / 1 (2 / 3 with the normals of quadrilateral cells) when
   // the caller's edges are all of one kind, else 4: one flux code path for i-
   // and j-edges, so that a wave holding both kinds runs it once
   constexpr int DIR = KIND < 0 ? 4 : (GEOM ? 2 : 0) + KIND;
   s.ax = idir ? 0 : 1;
-  if constexpr (GEOM) {
-    const size_t gc = (size_t)(ci + a.nh - 1) + (size_t)(cj + a.nh - 1) * (size_t)a.quad_ncx;
-    const size_t n = (size_t)a.quad_n;
-    s.nx = (R)global(a.quad)[(idir ? Q_NRX : Q_NTX) * n + gc];
-    s.ny = (R)global(a.quad)[(idir ? Q_NRY : Q_NTY) * n + gc];
-  } else {
-    s.nx = idir ? R(1) : R(0);
-    s.ny = idir ? R(0) : R(1);
-  }
+  edge_normal<GEOM>(a, idir, ci, cj, s);
   edge_flux<R, FLUX, DIR, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2]), a.low_mach_fix, s, pn, f, &sb);
   return true;
 }
@@ -438,41 +470,24 @@ __device__ inline void edge_pass(Args &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &
   }
 }
 
-// One tile of one stage.  Writes the block's CFL partial and sanity flags to
-// a.block_min[tile] / a.block_err[tile] when requested.  OUTFLOW_COL: the tile
-// also writes the +x outflow ghost column of the new state (the batched
-// kernel); the single-solve launch leaves that to k_outflow_column, since the
-// extra epilogue slows every tile of the fused kernel by ~5%.
-template <int FLUX, int LIMC, typename R, int TX, int TY, bool OUTFLOW_COL = false, bool GEOM = false,
-          int NT = kThreads, bool SPLIT = false, class Args>
-__device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm,
-                                  RedSmemT<NT / 64> &red) {
+// Phase 1 of a stage tile: the primitives of the tile and its halo into sp, ghost
+// cells through the boundary map.  Adds 1 to err where a checked cell holds a NaN;
+// returns whether every cell this thread loaded keeps the FastOps operations of
+// the reconstruction and of the flux (where it has a FastOps path) in range
+// (fast_ops_cell).  TVD2 under a flux without one divides too little for the
+// range vote to pay.
+template <int FLUX, int LIMC, typename R> constexpr bool fast_scheme() {
+  return !std::is_same<R, f32x>::value && (fast_ops_flux<FLUX>() || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
+}
+template <int FLUX, int LIMC, typename R, int TX, int TY, int NT, class Args, class Sp>
+__device__ inline bool load_tile(Args &a, int i0, int j0, Sp &sp, int &err) {
   constexpr int H = halo_of<LIMC>();
   constexpr int RX = TX + 2 * H, RY = TY + 2 * H;
-  // FP64 form: the reference's arithmetic bit for bit; precision form (f32x):
-  // a lighter FP64 epilogue (reciprocal-based primitive recovery and flux balance)
-  constexpr bool kExact = !std::is_same<R, f32x>::value;
-  auto &sp = sm.sp;
-  auto &sfi = sm.sfi;
-  auto &sfj = sm.sfj;
-  auto &red_min = red.m;
-  auto &red_err = red.e;
-  const int tid = threadIdx.x;
-  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
-  const int i0 = tx * TX + 1, j0 = ty * TY + 1;
-  const int ni = a.ni, nj = a.nj, nh = a.nh;
-  int err = 0;
-
-  // ---- 1. primitives of the tile + halo ---------------------------------
-  // (precision form outside MODE_RESIDUAL: recovered from U_k, and checked
-  // for NaN here, since no earlier stage stored and checked them)
-  const bool recover = !kExact && a.mode != MODE_RESIDUAL;
-  // FP64: whether every cell the edges read keeps the FastOps operations of the
-  // reconstruction and of the flux (where it has a FastOps path) in range
-  // (fast_ops_cell).  TVD2 under a flux without one divides too little for the
-  // range vote to pay.
-  constexpr bool kFastScheme =
-      kExact && (fast_ops_flux<FLUX>() || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
+  constexpr bool kFastScheme = fast_scheme<FLUX, LIMC, R>();
+  const int tid = threadIdx.x, ni = a.ni, nj = a.nj, nh = a.nh;
+  // precision form outside MODE_RESIDUAL: recovered from U_k, and checked
+  // for NaN here, since no earlier stage stored and checked them
+  const bool recover = std::is_same<R, f32x>::value && a.mode != MODE_RESIDUAL;
   bool in_range = true;
   // A tile whose halo lies inside the domain (all but the tiles along its
   // sides) reads its cells directly, without the boundary map
@@ -516,6 +531,175 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
       sp[3][ly][lx] = (R)pr.p;
     }
   }
+  return in_range;
+}
+
+// Geometry of one cell as the epilogue takes it: widths, edge lengths (bottom,
+// right, top, left), volume and its reciprocal (FP64: the exact one of a power of
+// two, else 0; precision form: rounded).
+struct CellGeo {
+  double dxv, dyv, lb, lr, lt, ll, vol, inv_vol;
+  bool pow2;
+};
+template <bool kExact, bool GEOM, class Args> __device__ inline CellGeo cell_geometry(Args &a, int gi, int gj) {
+  const int nh = a.nh;
+  const double EPSD = Lim<double>::eps;
+  double dxv, dyv, lb, lr, lt, ll, vol, inv_vol;
+  bool pow2;
+  if (!GEOM && a.ugeom) {
+    // uniform rectilinear grid: the same values, computed once on the host
+    dxv = a.ug[0];
+    dyv = a.ug[1];
+    lb = a.ug[2];
+    lr = a.ug[3];
+    lt = a.ug[4];
+    ll = a.ug[5];
+    vol = a.ug[6];
+    pow2 = a.ugeom_pow2 != 0;
+    inv_vol = kExact ? a.ug[7] : rcp64(vol);
+  } else {
+    if constexpr (GEOM) {
+      // quad_cell geometry of the cell: min_dx / min_dy, bottom / right / top / left lengths, volume
+      const size_t gc = (size_t)(gi + nh - 1) + (size_t)(gj + nh - 1) * (size_t)a.quad_ncx;
+      const size_t n = (size_t)a.quad_n;
+      dxv = global(a.quad)[Q_MDX * n + gc];
+      dyv = global(a.quad)[Q_MDY * n + gc];
+      lb = global(a.quad)[Q_LEN0 * n + gc];
+      lr = global(a.quad)[Q_LEN1 * n + gc];
+      lt = global(a.quad)[Q_LEN2 * n + gc];
+      ll = global(a.quad)[Q_LEN3 * n + gc];
+      vol = global(a.quad)[Q_VOL * n + gc];
+    } else {
+      dxv = global(a.dxi)[gi + nh - 1];
+      dyv = global(a.dyj)[gj + nh - 1];
+      double l1 = global(a.lxi)[gi + nh - 1], l2 = global(a.lyj)[gj + nh - 1];
+      // edge-length equalisation (quad_cell.f90:110-112) over (l1, l2, l1, l2)
+      double mx = fmax2(l1, l2), mn = fmin2(l1, l2);
+      lb = l1, lr = l2, lt = l1, ll = l2;
+      if (mx - mn < 2.0 * EPSD) lb = lr = lt = ll = mx;
+      vol = dxv * dyv;
+    }
+    uint64_t vb = (uint64_t)__double_as_longlong(vol);
+    const uint64_t ve = (vb >> 52) & 0x7FF;
+    pow2 = (vb & 0x000FFFFFFFFFFFFFull) == 0 && ve > 1 && ve < 2046;
+    // 1 / 2^k = 2^-k exactly: the sign of vol with the biased exponent 2046 - ve
+    const double inv_pow2 = __longlong_as_double((long long)((vb & 0x8000000000000000ull) | ((2046 - ve) << 52)));
+    inv_vol = kExact ? (pow2 ? inv_pow2 : 0.0) : rcp64(vol);
+  }
+  return CellGeo{dxv, dyv, lb, lr, lt, ll, vol, inv_vol, pow2};
+}
+
+// d/dt of one variable of a cell from its edge fluxes (right, left, top, bottom).
+// Precision form: the same FP64 flux balance without the reference's
+// max-normalisation and flushes (they only shape rounding at 1e-16); on a
+// rectilinear grid the right and left lengths are equal, as are the top and bottom
+// ones, so each pair takes one product with the length over the volume (the
+// difference of two binary32 fluxes is exact in FP64).
+template <bool kExact, bool GEOM>
+__device__ inline double flux_balance(const CellGeo &g, double Fi, double Fim, double Gj, double Gjm) {
+  if constexpr (kExact)
+    return divergence(Fi, Fim, Gj, Gjm, g.lb, g.lr, g.lt, g.ll, g.vol, g.pow2, g.inv_vol);
+  else if constexpr (GEOM)
+    return -(((Fi * g.lr) - (Fim * g.ll)) + ((Gj * g.lt) - (Gjm * g.lb))) * g.inv_vol;
+  else
+    return -(((Fi - Fim) * (g.lr * g.inv_vol)) + ((Gj - Gjm) * (g.lb * g.inv_vol)));
+}
+
+// Stage combination of one variable: U_0 and U_k at the cell (each read only by
+// the modes that take it) and the rate L.  The field operators' sum (its epsilon
+// flush only shapes rounding at 1e-16, which the precision form leaves out as in
+// its flux balance).
+template <bool kExact, class Args, class U0, class Uk>
+__device__ inline double combine(Args &a, double L, double dt, U0 &&u0, Uk &&uk) {
+  auto sum = [](double x, double y) { return kExact ? op_add(x, y) : x + y; };
+  if (a.mode == MODE_RESIDUAL) return L;
+  if (a.mode == MODE_FIRST) return sum(uk(), L * (a.c * dt));
+  if (a.mode == MODE_BASE) return sum(u0(), L * (dt * a.c));
+  const double t = sum(u0() * a.a, uk() * a.b);
+  return sum(t, L * (a.c * dt));
+}
+
+// Primitives of a cell's new state nv for the next stage (assign_fluid ->
+// calculate_derived_quantities, mod_fluid.f90:564-591), its checks and, on the
+// last stage, its CFL value (else +inf).  Precision form: the next stage recovers
+// the primitives itself; only the last stage needs them here.
+template <bool kExact, bool OUTFLOW_COL = false, class Args>
+__device__ inline double finish_cell(Args &a, const double (&nv)[4], size_t off, int gi, const CellGeo &g, int &err) {
+  const size_t fs = (size_t)a.fstride;
+  double cs;
+  Prim<double> q = kExact ? cons_to_prim_vote(nv[0], nv[1], nv[2], nv[3], a.gamma, a.gamma - 1.0, &cs)
+                          : cons_to_prim_fast(nv[0], nv[1], nv[2], nv[3], a.gamma, a.gamma - 1.0, 1, &cs);
+  if (kExact) {
+    st_cell<kExact>(&a.prim_out[0][off], q.rho);
+    st_cell<kExact>(&a.prim_out[0][off + fs], q.u);
+    st_cell<kExact>(&a.prim_out[0][off + 2 * fs], q.v);
+    st_cell<kExact>(&a.prim_out[0][off + 3 * fs], q.p);
+  }
+  if (kExact && OUTFLOW_COL && gi == a.ni && a.bc[0] == BC_OUTFLOW) {
+    Prim<double> o = outflow_ghost(q, a.gamma, a.bc_pressure);
+    global(a.prim_out[0])[off + 1] = o.rho;
+    global(a.prim_out[0])[off + fs + 1] = o.u;
+    global(a.prim_out[0])[off + 2 * fs + 1] = o.v;
+    global(a.prim_out[0])[off + 3 * fs + 1] = o.p;
+  }
+  if (q.rho != q.rho || q.u != q.u || q.v != q.v || q.p != q.p) err |= 1;
+  if (!a.last_stage) return __builtin_inf();
+  if (q.rho < 0.0) err |= 2;
+  if (q.p < 0.0) err |= 4;
+  // get_timestep (mod_fluid.f90:554-558); min_dx/min_dy = |dx|, |dy| on rectilinear cells
+  // (quad cells: the non-negative min_dx / min_dy themselves)
+  return a.cfl / (((absd(q.u) + cs) / absd(g.dxv)) + ((absd(q.v) + cs) / absd(g.dyv)));
+}
+
+// The tile's CFL minimum and sanity flags, reduced over the workgroup.
+template <int NT, class Args>
+__device__ inline void store_tile_result(Args &a, int tile, double lmin, int err, RedSmemT<NT / 64> &red) {
+  const int tid = threadIdx.x;
+  const double wm = wave_min(lmin);
+  const int we = wave_or(err);
+  if ((tid & 63) == 0) {
+    red.m[tid >> 6] = wm;
+    red.e[tid >> 6] = we;
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  double m = red.m[0];
+  int e = red.e[0];
+#pragma unroll
+  for (int k = 1; k < NT / 64; ++k) {
+    m = (red.m[k] < m) ? red.m[k] : m;
+    e |= red.e[k];
+  }
+  if (a.last_stage) global(a.block_min)[tile] = m;
+  if (a.err_assign)
+    global(a.block_err)[tile] = (a.err_prev ? global(a.err_prev)[tile] : 0) | e;
+  else if (a.block_err && e)
+    global(a.block_err)[tile] |= e;
+}
+
+// One tile of one stage.  Writes the block's CFL partial and sanity flags to
+// a.block_min[tile] / a.block_err[tile] when requested.  OUTFLOW_COL: the tile
+// also writes the +x outflow ghost column of the new state (the batched
+// kernel); the single-solve launch leaves that to k_outflow_column, since the
+// extra epilogue slows every tile of the fused kernel by ~5%.
+template <int FLUX, int LIMC, typename R, int TX, int TY, bool OUTFLOW_COL = false, bool GEOM = false,
+          int NT = kThreads, bool SPLIT = false, class Args>
+__device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &sm,
+                                  RedSmemT<NT / 64> &red) {
+  // FP64 form: the reference's arithmetic bit for bit; precision form (f32x):
+  // a lighter FP64 epilogue (reciprocal-based primitive recovery and flux balance)
+  constexpr bool kExact = !std::is_same<R, f32x>::value;
+  auto &sfi = sm.sfi;
+  auto &sfj = sm.sfj;
+  const int tid = threadIdx.x;
+  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+  const int i0 = tx * TX + 1, j0 = ty * TY + 1;
+  const int ni = a.ni, nj = a.nj;
+  int err = 0;
+
+  // ---- 1. primitives of the tile + halo ---------------------------------
+  constexpr bool kFastScheme = fast_scheme<FLUX, LIMC, R>();
+  const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT>(a, i0, j0, sm.sp, err);
   if constexpr (kFastScheme) {
     const int vote = __all(in_range ? 1 : 0);
     if ((tid & 63) == 0) red.fast[tid >> 6] = vote;
@@ -554,53 +738,11 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
   double csq[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) csq[v] = 0.0;
-  const double EPSD = Lim<double>::eps;
   for (int c = tid; c < TX * TY; c += NT) {
     int cy = c / TX, cx = c - cy * TX;
     int gi = i0 + cx, gj = j0 + cy;
     if (gi > ni || gj > nj) continue;
-    double dxv, dyv, lb, lr, lt, ll, vol, inv_vol;
-    bool pow2;
-    if (!GEOM && a.ugeom) {
-      // uniform rectilinear grid: the same values, computed once on the host
-      dxv = a.ug[0];
-      dyv = a.ug[1];
-      lb = a.ug[2];
-      lr = a.ug[3];
-      lt = a.ug[4];
-      ll = a.ug[5];
-      vol = a.ug[6];
-      pow2 = a.ugeom_pow2 != 0;
-      inv_vol = kExact ? a.ug[7] : rcp64(vol);
-    } else {
-      if constexpr (GEOM) {
-        // quad_cell geometry of the cell: min_dx / min_dy, bottom / right / top / left lengths, volume
-        const size_t gc = (size_t)(gi + nh - 1) + (size_t)(gj + nh - 1) * (size_t)a.quad_ncx;
-        const size_t n = (size_t)a.quad_n;
-        dxv = global(a.quad)[Q_MDX * n + gc];
-        dyv = global(a.quad)[Q_MDY * n + gc];
-        lb = global(a.quad)[Q_LEN0 * n + gc];
-        lr = global(a.quad)[Q_LEN1 * n + gc];
-        lt = global(a.quad)[Q_LEN2 * n + gc];
-        ll = global(a.quad)[Q_LEN3 * n + gc];
-        vol = global(a.quad)[Q_VOL * n + gc];
-      } else {
-        dxv = global(a.dxi)[gi + nh - 1];
-        dyv = global(a.dyj)[gj + nh - 1];
-        double l1 = global(a.lxi)[gi + nh - 1], l2 = global(a.lyj)[gj + nh - 1];
-        // edge-length equalisation (quad_cell.f90:110-112) over (l1, l2, l1, l2)
-        double mx = fmax2(l1, l2), mn = fmin2(l1, l2);
-        lb = l1, lr = l2, lt = l1, ll = l2;
-        if (mx - mn < 2.0 * EPSD) lb = lr = lt = ll = mx;
-        vol = dxv * dyv;
-      }
-      uint64_t vb = (uint64_t)__double_as_longlong(vol);
-      const uint64_t ve = (vb >> 52) & 0x7FF;
-      pow2 = (vb & 0x000FFFFFFFFFFFFFull) == 0 && ve > 1 && ve < 2046;
-      // 1 / 2^k = 2^-k exactly: the sign of vol with the biased exponent 2046 - ve
-      const double inv_pow2 = __longlong_as_double((long long)((vb & 0x8000000000000000ull) | ((2046 - ve) << 52)));
-      inv_vol = kExact ? (pow2 ? inv_pow2 : 0.0) : rcp64(vol);
-    }
+    const CellGeo g = cell_geometry<kExact, GEOM>(a, gi, gj);
     size_t off = (size_t)(gj - 1) * a.pitch + (size_t)(gi - 1);
     const size_t fs = (size_t)a.fstride;
     double fst[4] = {0.0, 0.0, 0.0, 0.0};  // issued before the flux balance to hide their latency
@@ -608,8 +750,6 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
 #pragma unroll
       for (int v = 0; v < 4; ++v) fst[v] = global(a.conv_first[0])[off + v * fs];
     }
-    // precision form, rectilinear cells (lr == ll, lt == lb): lengths over the volume
-    const double sx = kExact ? 0.0 : lr * inv_vol, sy = kExact ? 0.0 : lb * inv_vol;
     double nv[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -622,36 +762,12 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
         Gj = (double)sfj[v][cy + 1][cx];
         Gjm = (double)sfj[v][cy][cx];
       }
-      double L;
-      if constexpr (kExact) {
-        L = divergence(Fi, Fim, Gj, Gjm, lb, lr, lt, ll, vol, pow2, inv_vol);
-      } else {
-        // precision form: the same FP64 flux balance without the reference's
-        // max-normalisation and flushes (they only shape rounding at 1e-16); on
-        // a rectilinear grid the right and left lengths are equal, as are the
-        // top and bottom ones, so each pair takes one product (the difference of
-        // two binary32 fluxes is exact in FP64)
-        if constexpr (GEOM)
-          L = -(((Fi * lr) - (Fim * ll)) + ((Gj * lt) - (Gjm * lb))) * inv_vol;
-        else
-          L = -(((Fi - Fim) * sx) + ((Gj - Gjm) * sy));
-      }
+      double L = flux_balance<kExact, GEOM>(g, Fi, Fim, Gj, Gjm);
       // time_derivative's energy source (mod_fluid.f90:500-509): a plain sum
       if (v == 3 && a.src_E) L = L + global(a.src_E)[off];
-      // the field operators' sum (its epsilon flush only shapes rounding at 1e-16,
-      // which the precision form leaves out as in its flux balance)
-      auto sum = [](double x, double y) { return kExact ? op_add(x, y) : x + y; };
-      double r;
-      if (a.mode == MODE_RESIDUAL) {
-        r = L;
-      } else if (a.mode == MODE_FIRST) {
-        r = sum(global(a.uk[0])[off + v * fs], L * (a.c * dt));
-      } else if (a.mode == MODE_BASE) {
-        r = sum(ld_cell<kExact>(&a.u0[0][off + v * fs]), L * (dt * a.c));
-      } else {
-        double t = sum(ld_cell<kExact>(&a.u0[0][off + v * fs]) * a.a, global(a.uk[0])[off + v * fs] * a.b);
-        r = sum(t, L * (a.c * dt));
-      }
+      const double r = combine<kExact>(
+          a, L, dt, [&] { return ld_cell<kExact>(&a.u0[0][off + v * fs]); },
+          [&] { return global(a.uk[0])[off + v * fs]; });
       nv[v] = r;
       if (conv) {
         double d = r - fst[v];
@@ -661,36 +777,9 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
       st_cell<kExact>(&a.out[0][off + v * fs], r);
     }
     if (a.mode == MODE_RESIDUAL) continue;
-    // precision form: the next stage recovers the primitives of this state
-    // itself; only the last stage needs them here (checks and CFL)
     if (!kExact && !a.last_stage) continue;
-    // primitives of the new state for the next stage (assign_fluid ->
-    // calculate_derived_quantities, mod_fluid.f90:564-591) and its NaN check
-    double cs;
-    Prim<double> q = kExact ? cons_to_prim_vote(nv[0], nv[1], nv[2], nv[3], a.gamma, a.gamma - 1.0, &cs)
-                            : cons_to_prim_fast(nv[0], nv[1], nv[2], nv[3], a.gamma, a.gamma - 1.0, 1, &cs);
-    if (kExact) {
-      st_cell<kExact>(&a.prim_out[0][off], q.rho);
-      st_cell<kExact>(&a.prim_out[0][off + fs], q.u);
-      st_cell<kExact>(&a.prim_out[0][off + 2 * fs], q.v);
-      st_cell<kExact>(&a.prim_out[0][off + 3 * fs], q.p);
-    }
-    if (kExact && OUTFLOW_COL && gi == ni && a.bc[0] == BC_OUTFLOW) {
-      Prim<double> g = outflow_ghost(q, a.gamma, a.bc_pressure);
-      global(a.prim_out[0])[off + 1] = g.rho;
-      global(a.prim_out[0])[off + fs + 1] = g.u;
-      global(a.prim_out[0])[off + 2 * fs + 1] = g.v;
-      global(a.prim_out[0])[off + 3 * fs + 1] = g.p;
-    }
-    if (q.rho != q.rho || q.u != q.u || q.v != q.v || q.p != q.p) err |= 1;
-    if (a.last_stage) {
-      if (q.rho < 0.0) err |= 2;
-      if (q.p < 0.0) err |= 4;
-      // get_timestep (mod_fluid.f90:554-558); min_dx/min_dy = |dx|, |dy| on rectilinear cells
-      // (quad cells: the non-negative min_dx / min_dy themselves)
-      double val = a.cfl / (((absd(q.u) + cs) / absd(dxv)) + ((absd(q.v) + cs) / absd(dyv)));
-      lmin = (val < lmin) ? val : lmin;
-    }
+    const double val = finish_cell<kExact, OUTFLOW_COL>(a, nv, off, gi, g, err);
+    lmin = (val < lmin) ? val : lmin;
   }
 
   if (conv) {
@@ -709,27 +798,7 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
     }
   }
 
-  if (a.last_stage || a.block_err) {
-    double wm = wave_min(lmin);
-    int we = wave_or(err);
-    int w = tid >> 6;
-    if ((tid & 63) == 0) {
-      red_min[w] = wm;
-      red_err[w] = we;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      double m = red_min[0];
-      int e = red_err[0];
-#pragma unroll
-      for (int k = 1; k < NT / 64; ++k) {
-        m = (red_min[k] < m) ? red_min[k] : m;
-        e |= red_err[k];
-      }
-      if (a.block_min) global(a.block_min)[tile] = m;
-      if (a.block_err && e) global(a.block_err)[tile] |= e;
-    }
-  }
+  if (a.last_stage || a.block_err) store_tile_result<NT>(a, tile, lmin, err, red);
 }
 
 // Single-solve stage launch: one workgroup per tile, XCD-aware tile order.
