@@ -514,6 +514,27 @@ static __global__ void k_apply_bc(FieldGeom g, int ld, double *rho, double *u, d
   p[d] = q.p;
 }
 
+// The ghost cells of four halo'd fields (n elements each), field after field: the
+// nh rows below the interior, the nh cells left and right of each interior row,
+// the nh rows above.
+__host__ __device__ inline int ghost_count(int ni, int nj, int nh) { return 2 * nh * (ni + 2 * nh) + 2 * nh * nj; }
+__host__ __device__ inline size_t ghost_cell(int k, int ni, int nj, int nh, int ld) {
+  const int nx = ni + 2 * nh, low = nh * nx, mid = 2 * nh * nj;
+  if (k < low) return (size_t)(k % nx) + (size_t)(k / nx) * ld;
+  if (k < low + mid) {
+    const int q = (k - low) % (2 * nh), row = (k - low) / (2 * nh);
+    return (size_t)(q < nh ? q : q + ni) + (size_t)(row + nh) * ld;
+  }
+  k -= low + mid;
+  return (size_t)(k % nx) + (size_t)(k / nx + nh + nj) * ld;
+}
+static __global__ void k_pack_ghosts(FieldGeom g, int ld, size_t n, const double *__restrict__ fields,
+                                     double *__restrict__ ghosts) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, m = ghost_count(g.ni, g.nj, g.nh);
+  if (k >= m) return;
+  ghosts[(size_t)blockIdx.y * m + k] = fields[blockIdx.y * n + ghost_cell(k, g.ni, g.nj, g.nh, ld)];
+}
+
 // muscl_interpolation_t%interpolate_edge_values on a halo'd field q:
 // edges (2, 0:ni, 0:nj) for both directions.
 template <typename R, int LIMC>
