@@ -14,7 +14,7 @@ struct FieldGeom {
   int ni, nj, nh, pitch;
   int bc[4];
   double gamma, cfl;
-  double gas[3];  // gas_constants(gamma)
+  double gas[4];  // gas_constants(gamma)
   double bc_pressure;
   const double *dxi, *dyj;
   const double *quad;  // per-cell quad_cell geometry (QuadSlot arrays), null on rectilinear grids
@@ -607,7 +607,7 @@ static __global__ void k_edge_flux(FieldGeom g, int ld, const double *__restrict
   pn.p00 = P(0, 0); pn.p10 = P(1, 0); pn.p20 = P(2, 0); pn.pm10 = P(-1, 0);
   pn.p0p = P(0, 1); pn.p0m = P(0, -1); pn.p1p = P(1, 1); pn.p1m = P(1, -1);
   R f[4];
-  const Gas<R> gas = gas_of<R>(g.gamma, g.gas[0], g.gas[1], g.gas[2]);
+  const Gas<R> gas = gas_of<R>(g.gamma, g.gas[0], g.gas[1], g.gas[2], g.gas[3]);
   if (g.quad) {  // normal of the right (i-edge) or top (j-edge) edge of cell (i, j)
     const size_t gc = (size_t)(i + g.nh - 1) + (size_t)(j + g.nh - 1) * (size_t)g.quad_ncx;
     const size_t n = (size_t)g.quad_n;

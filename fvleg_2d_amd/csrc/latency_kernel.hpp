@@ -100,7 +100,7 @@ __device__ inline void latency_edges(Args &a, Smem &sm, int i0, int j0) {
     s.ax = idir ? 0 : 1;
     edge_normal<GEOM>(a, idir, ci, cj, s);
     R f[4];
-    edge_flux<R, FLUX, 4, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2]), a.low_mach_fix, s, pn, f, &sb);
+    edge_flux<R, FLUX, 4, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2], a.gas[3]), a.low_mach_fix, s, pn, f, &sb);
 #pragma unroll
     for (int v = 0; v < 4; ++v) sm.lr[0][v][0][e] = f[v];
   }

@@ -132,13 +132,12 @@ __device__ inline Prim<double> cons_to_prim(double r, double ru, double rv, doub
   return Prim<double>{r, u, v, p};
 }
 
-// 1/x in FP64 to about 1 ulp: hardware estimate plus two Newton steps (the
+// 1/x in FP64 to about 1 ulp: hardware estimate plus one third-order step (the
 // precision form's epilogue; the FP64 form divides).
 __device__ inline double rcp64(double x) {
-  double r = __builtin_amdgcn_rcp(x);
+  const double r = __builtin_amdgcn_rcp(x);
   double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
+  e = __builtin_fma(e, e, e);
   return __builtin_fma(r, e, r);
 }
 
@@ -162,9 +161,10 @@ __device__ inline Prim<double> cons_to_prim_fast(double r, double ru, double rv,
 // the quotient with one correction (v_div_fmas) and a special-case fix-up
 // (v_div_fixup); sqrt(x) to an input scaling below 2^-767, v_rsq, Goldschmidt
 // steps, the inverse scaling and a select for 0 / inf.  While the scalings are
-// identities and no special case arises, dropping those steps leaves the same
-// operations on the same values, hence the same bits.  FastOps is that
-// remainder, with the reciprocal of a shared denominator formed once.  The
+// identities and no special case arises, what is left without those steps gives
+// the same bits: a quotient corrected once from a rounded reciprocal is the
+// rounded quotient.  FastOps is that remainder, with the reciprocal of a shared
+// denominator formed once.  The
 // stage kernel uses it only on tiles whose operands keep every division in
 // range (numerator 0 or |a| >= 2^-969, 2^-1021 <= |b| < 2^1021, normal
 // quotient, exponents less than 768 apart; square roots of 2^-767 <= x < inf)
@@ -174,6 +174,7 @@ __device__ inline Prim<double> cons_to_prim_fast(double r, double ru, double rv,
 struct IeeeOps {
   template <typename T> struct Rcp { T b; };
   template <typename T> static __device__ Rcp<T> rcp(T b) { return Rcp<T>{b}; }
+  template <typename T> static __device__ Rcp<T> rcp_of(T b, T) { return Rcp<T>{b}; }
   template <typename T> static __device__ T div(T a, Rcp<T> r) { return a / r.b; }
   template <typename T> static __device__ T div(T a, T b) { return a / b; }
   template <typename T> static __device__ T sqrt_pos(T x) { return sqrtr(x); }
@@ -183,14 +184,18 @@ struct IeeeOps {
 };
 struct FastOps {
   template <typename T> struct Rcp { double b, y; };
+  // v_rcp_f64 is within 2^-24.3 (measured over a binade), so one third-order step,
+  // y (1 + e + e^2) with e = 1 - b y exact to 2^-77, is within 2^-72 before its last
+  // rounding: the rounded reciprocal except where that lies within 2^-19 ulp of a
+  // tie, in three operations where two Newton steps take four.
   static __device__ Rcp<double> rcp(double b) {
-    double y = __builtin_amdgcn_rcp(b);
+    const double y = __builtin_amdgcn_rcp(b);
     double e = __builtin_fma(-b, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-b, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    return Rcp<double>{b, y};
+    e = __builtin_fma(e, e, e);
+    return Rcp<double>{b, __builtin_fma(y, e, y)};
   }
+  // y = 1 / b formed once, correctly rounded
+  static __device__ Rcp<double> rcp_of(double b, double y) { return Rcp<double>{b, y}; }
   static __device__ double div(double a, Rcp<double> r) {
     const double q = a * r.y;
     const double e = __builtin_fma(-r.b, q, a);
@@ -298,10 +303,21 @@ __device__ inline Prim<double> cons_to_prim_vote(double r, double ru, double rv,
 // Reconstruction (edge states L/R at the interface between cells 0 and 1).
 // Stencil values along the edge normal: qm3=q(-2), qm=q(-1), q0, q1, q2, q3=q(+3).
 // ---------------------------------------------------------------------------
+//
+// half_phi: phi(r) / 2, exact.  On FastOps tiles r is finite, so the hardware min
+// and max give the compare-and-select's values, and van Leer's numerator r + |r|
+// (0 or 2 r, exactly) is halved before the division instead of the quotient after.
 template <typename R, class D = IeeeOps> __device__ inline R tvd_phi(int lim, R r) {
   if (lim == LIM_MINMOD) return fmax2(R(0), fmin2(r, R(1)));  // muscl_tvd2.fypp:196
   if (lim == LIM_SUPERBEE) return fmax2(fmax2(R(0), fmin2(R(2) * r, R(1))), fmin2(r, R(2)));  // :198
   return D::div(r + absd(r), R(1) + absd(r));  // :200 (numerator +0 or positive)
+}
+
+template <int LIMC, class D> __device__ inline double half_phi(double r) {
+  if constexpr (!std::is_same<D, FastOps>::value) return 0.5 * tvd_phi<double, D>(LIMC, r);
+  else if constexpr (LIMC == LIM_MINMOD) return 0.5 * D::max(0.0, D::min(r, 1.0));
+  else if constexpr (LIMC == LIM_SUPERBEE) return 0.5 * D::max(D::max(0.0, D::min(2.0 * r, 1.0)), D::min(r, 2.0));
+  else return D::div(D::max(r, 0.0), 1.0 + absd(r));
 }
 
 // Precision form: phi(b / (a + 1e-16)) * a, the limited slope, written without
@@ -334,10 +350,8 @@ __device__ inline void recon_tvd2(R qm, R q0, R q1, R q2, R &L, R &Rv) {
   } else {
     R r_L = D::div(dp, dm + R(1e-16));
     R r_R = D::div(dp, d3 + R(1e-16));
-    R phi = tvd_phi<R, D>(LIMC, r_L);
-    L = q0 + R(0.5) * phi * dm;
-    phi = tvd_phi<R, D>(LIMC, r_R);
-    Rv = q1 - R(0.5) * phi * d3;
+    L = q0 + half_phi<LIMC, D>(r_L) * dm;
+    Rv = q1 - half_phi<LIMC, D>(r_R) * d3;
   }
 }
 
@@ -429,19 +443,20 @@ template <typename R> struct PressNbr {
 // Constants of the ideal-gas law the fluxes take, formed once per solve on the
 // host in FP64 (gas_constants) instead of on every edge: gamma / (gamma - 1),
 // 2 ((gamma - 1) / (gamma + 1)) (which equals (2 (gamma - 1)) / (gamma + 1): a
-// product by 2 is exact) and (gamma + 1) / (2 gamma), each one IEEE operation
+// product by 2 is exact), (gamma + 1) / (2 gamma) and 1 / (gamma - 1), each one IEEE operation
 // sequence on gamma, so the FP64 values are the bits the per-edge formulas
 // gave.  The precision form rounds them to binary32.
 template <typename R> struct Gas {
-  R gamma, gg, cr2, hf;
+  R gamma, gg, cr2, hf, inv_gm1;
 };
-__host__ __device__ inline void gas_constants(double gamma, double out[3]) {
+__host__ __device__ inline void gas_constants(double gamma, double out[4]) {
   out[0] = gamma / (gamma - 1.0);
   out[1] = 2.0 * ((gamma - 1.0) / (gamma + 1.0));
   out[2] = (gamma + 1.0) / (2.0 * gamma);
+  out[3] = 1.0 / (gamma - 1.0);
 }
-template <typename R> __device__ inline Gas<R> gas_of(double gamma, double gg, double cr2, double hf) {
-  return Gas<R>{R(gamma), R(gg), R(cr2), R(hf)};
+template <typename R> __device__ inline Gas<R> gas_of(double gamma, double gg, double cr2, double hf, double inv_gm1) {
+  return Gas<R>{R(gamma), R(gg), R(cr2), R(hf), R(inv_gm1)};
 }
 
 // SLAU family: slau_solver.fypp:355-490.  With D = FastOps: every numerator is
@@ -498,10 +513,19 @@ __device__ inline void flux_slau(const Gas<R> &gas, const EdgeState<R> &s, const
   R rho_bar = R(0.5) * (rho_L + rho_R);
   R M_plus = over_c(V_n_plus);
   R M_minus = over_c(V_n_minus);
-  R Beta_plus = (absd(M_plus) < R(1)) ? R(0.25) * (R(2) - M_plus) * sq(M_plus + R(1))
-                                       : R(0.5) * (R(1) + copysignr(R(1), M_plus));
-  R Beta_minus = (absd(M_minus) < R(1)) ? R(0.25) * (R(2) + M_minus) * sq(M_minus - R(1))
-                                         : R(0.5) * (R(1) + copysignr(R(1), -M_minus));
+  // for |M| >= 1 the split of M clamped to [-1, 1] is exactly the supersonic value
+  // 1 or 0 (FastOps: M is finite)
+  R Beta_plus, Beta_minus;
+  if constexpr (std::is_same<D, FastOps>::value) {
+    const R Mp = D::max(D::min(M_plus, R(1)), R(-1)), Mm = D::max(D::min(M_minus, R(1)), R(-1));
+    Beta_plus = R(0.25) * (R(2) - Mp) * sq(Mp + R(1));
+    Beta_minus = R(0.25) * (R(2) + Mm) * sq(Mm - R(1));
+  } else {
+    Beta_plus = (absd(M_plus) < R(1)) ? R(0.25) * (R(2) - M_plus) * sq(M_plus + R(1))
+                                      : R(0.5) * (R(1) + copysignr(R(1), M_plus));
+    Beta_minus = (absd(M_minus) < R(1)) ? R(0.25) * (R(2) + M_minus) * sq(M_minus - R(1))
+                                        : R(0.5) * (R(1) + copysignr(R(1), -M_minus));
+  }
   R delta_p = p_R - p_L;
   if (absd(delta_p) < eps || absd(delta_p) < THRESHOLD * p_bar) delta_p = R(0);
   R delta_rho = rho_R - rho_L;
@@ -587,6 +611,16 @@ template <typename R> __device__ inline R pw_M_minus(R M) {
   return -(R(0.25) * sq(M - R(1)));
 }
 
+// min(p_L / p_R, p_R / p_L).  FP64: of two positive finite pressures the smaller
+// over the larger, since rounding keeps both quotients on their side of 1.
+template <typename R> __device__ inline R pw_ratio(R p_L, R p_R) {
+  if constexpr (std::is_same<R, double>::value) {
+    const R lo = fmin2(p_L, p_R), hi = fmax2(p_L, p_R);
+    if (lo > R(0) && hi <= R(1.7976931348623157e308)) return lo / hi;
+  }
+  return fmin2((p_L / p_R), (p_R / p_L));
+}
+
 template <typename R, int DIR>
 __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const EdgeState<R> &s, const PressNbr<R> &pn,
                                    R out[4]) {
@@ -622,7 +656,7 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
   R P_R_minus = pw_P_minus(M_R);
   R P_L_plus = pw_P_plus(M_L);
   R p_s = p_L * P_L_plus + p_R * P_R_minus;
-  R mt = fmin2((p_L / p_R), (p_R / p_L));
+  R mt = pw_ratio(p_L, p_R);
   R w = R(1) - mt * mt * mt;
   // get_f neighbours (ausmpw_plus_solver.fypp:433-441): i-dir p1=(0,-1),(1,-1) p2=(0,+1),(1,+1);
   // j-dir p1=(i+1,j),(i+1,j+1) p2=(i-1,j),(i-1,j+1), i.e. transverse +1 then -1.
@@ -657,7 +691,12 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
 
 // Roe (reference variant): roe_solver.fypp:420-511, f_h 519-527
 template <typename R> __device__ inline R roe_f_h(R pL, R pR) {
-  R ratio = absd(pR - pL) / (fmin2(pR, pL) + R(1e-16));
+  const R a = absd(pR - pL), b = fmin2(pR, pL) + R(1e-16);
+  // FP64: the rounded quotient a / b is below 1 exactly where a < b or b < 0
+  // (a >= 0; neighbouring binary64 numbers differ by at least 2^-53 relative, so
+  // no a < b rounds up to 1; NaN and infinite operands compare alike)
+  if constexpr (std::is_same<R, double>::value) return (a < b || b < R(0)) ? R(0) : R(1);
+  const R ratio = a / b;
   return (ratio < R(1)) ? R(0) : R(1);
 }
 
@@ -754,9 +793,19 @@ __device__ inline void flux_ausm_plus(const Gas<R> &gas, const EdgeState<R> &s, 
   if (absd(M_sum) < R(1e-13)) M_sum = R(0);
   R M_half = M_sum + R(0);
   if (absd(M_half) < R(1e-13)) M_half = R(0);
-  R P_plus = (absd(M_L) >= R(1)) ? (R(0.5) * (M_L + absd(M_L))) / M_L
+  // supersonic: half (M + |M|) over M, which FP64 writes without the division: 1 or 0
+  // (NaN for an infinite M; the sign of a zero is lost in the sum below)
+  auto super_plus = [](R M) {
+    if constexpr (std::is_same<R, double>::value) return (M > R(0) ? R(1) : R(0)) + (M - M);
+    else return (R(0.5) * (M + absd(M))) / M;
+  };
+  auto super_minus = [](R M) {
+    if constexpr (std::is_same<R, double>::value) return (M < R(0) ? R(1) : R(0)) + (M - M);
+    else return (R(0.5) * (M - absd(M))) / M;
+  };
+  R P_plus = (absd(M_L) >= R(1)) ? super_plus(M_L)
                                   : M2p_L * ((R(2) - M_L) - R(16) * alpha * M_L * M2m_L);
-  R P_minus = (absd(M_R) >= R(1)) ? (R(0.5) * (M_R - absd(M_R))) / M_R
+  R P_minus = (absd(M_R) >= R(1)) ? super_minus(M_R)
                                    : M2m_R * ((R(-2) - M_R) + R(16) * alpha * M_R * M2p_R);
   R p_half = P_plus * p_L + P_minus * p_R + R(0);
   if (M_half > R(0)) {
@@ -801,7 +850,7 @@ __device__ inline void flux_hllc(const Gas<R> &gas, const EdgeState<R> &s, R out
   R mL = rL * (SL - qL);
   R mR = rR * (SR - qR);
   R S_star = D::div(pR - pL + qL * mL - qR * mR, mL - mR);
-  const auto d_gm1 = D::rcp(gm1);
+  const auto d_gm1 = D::rcp_of(gm1, gas.inv_gm1);
   R EL = D::div(pL, d_gm1) + R(0.5) * rL * (uL * uL + vL * vL);
   R ER = D::div(pR, d_gm1) + R(0.5) * rR * (uR * uR + vR * vR);
   if (R(0) <= SL) {
@@ -885,7 +934,7 @@ __device__ inline void flux_m_ausmpw(const Gas<R> &gas, int low_mach_fix, const 
   R P_R_minus = (absd(M_R) > R(1)) ? R(0.5) * (R(1) - copysignr(R(1), M_R)) : R(0.25) * sq(M_R - R(1)) * (R(2) + M_R);
   R P_L_plus = (absd(M_L) > R(1)) ? R(0.5) * (R(1) + copysignr(R(1), M_L)) : R(0.25) * sq(M_L + R(1)) * (R(2) - M_L);
   R p_s = p_L * P_L_plus + p_R * P_R_minus;
-  R mt = fmin2((p_L / p_R), (p_R / p_L));
+  R mt = pw_ratio(p_L, p_R);
   R w = R(1) - (mt * mt * mt);
   // get_f neighbours as AUSMPW+: i-dir p1 = (0,-1),(1,-1), p2 = (0,+1),(1,+1); j-dir the transverse +1 then -1
   R p1L = edge_ax0<R, DIR>(s) ? pn.p0m : pn.p0p, p1R = edge_ax0<R, DIR>(s) ? pn.p1m : pn.p1p;
@@ -973,17 +1022,33 @@ template <int FLUX> constexpr bool needs_pressure_nbrs() {
 }
 
 // qa = a / m and qb = b / m for m = max(|a|, |b|, 1) != 1.  A finite m is |a|
-// or |b| itself, and x / |x| is exactly copysign(1, x), so one IEEE division
-// gives both quotients bit for bit; inf / NaN operands keep both divisions.
+// or |b| itself, and x / |x| is exactly copysign(1, x), so one division gives both
+// quotients bit for bit.  Below 2^1000 it is the FastOps one: the other operand is
+// at most m, and where it is so small (below 2^-969) that the quotient's correction
+// loses bits, the quotient is lost beside the 1 anyway.  Larger m, inf and NaN keep
+// both IEEE divisions.
 __device__ inline void scaled_pair(double a, double b, double m, double &qa, double &qb) {
-  const bool a_big = absd(a) == m;
-  const double q = (a_big ? b : a) / m;
-  qa = a_big ? copysignr(1.0, a) : q;
-  qb = a_big ? q : copysignr(1.0, b);
-  if (!(m <= 1.7976931348623157e308)) {
+  if (!(m <= 0x1p1000)) {
     qa = a / m;
     qb = b / m;
+    return;
   }
+  const bool a_big = absd(a) == m;
+  const double q = FastOps::div(a_big ? b : a, m);
+  qa = a_big ? copysignr(1.0, a) : q;
+  qb = a_big ? q : copysignr(1.0, b);
+}
+
+// d / vol for a cell volume within [2^-400, 2^400] whose reciprocal the cell's four
+// variables share; |d| over 2^600, inf and NaN, and other volumes take the IEEE
+// division.  (A d below 2^-969 may lose its last bits: a rate that no sum keeps.)
+__device__ inline double over_volume(double d, const FastOps::Rcp<double> &vol) {
+  if (vol.y != 0.0 && absd(d) <= 0x1p600) return FastOps::div(d, vol);
+  return d / vol.b;
+}
+__device__ inline FastOps::Rcp<double> volume_rcp(double vol) {
+  const double av = absd(vol);
+  return FastOps::Rcp<double>{vol, (av >= 0x1p-400 && av <= 0x1p400) ? FastOps::rcp(vol).y : 0.0};
 }
 
 // ---------------------------------------------------------------------------
@@ -991,7 +1056,7 @@ __device__ inline void scaled_pair(double a, double b, double m, double &qa, dou
 // (flux_solver.f90:252-277 and 395-425).  l1..l4 = bottom/right/top/left lengths.
 // ---------------------------------------------------------------------------
 __device__ inline double divergence(double Fi, double Fim, double Gj, double Gjm, double l1, double l2, double l3,
-                                    double l4, double vol, bool vol_pow2, double inv_vol) {
+                                    double l4, const FastOps::Rcp<double> &vol, bool vol_pow2, double inv_vol) {
   const double REL_TOL = 1e-14;
   const double NEAR_ZERO = 5.0 * Lim<double>::tiny;
   // m = max(|F|, |Fm|, 1) by the hardware max (one instruction instead of a
@@ -1022,7 +1087,7 @@ __device__ inline double divergence(double Fi, double Fim, double Gj, double Gjm
   if (absd(fl) < NEAR_ZERO) fl = 0.0;
   double d = -fl;
   // x / 2^k is exactly x * 2^-k: skip the IEEE division for power-of-two volumes
-  return vol_pow2 ? d * inv_vol : d / vol;
+  return vol_pow2 ? d * inv_vol : over_volume(d, vol);
 }
 
 }  // namespace cato

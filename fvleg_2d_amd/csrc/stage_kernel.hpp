@@ -399,7 +399,7 @@ __device__ __forceinline__ bool tile_edge(Args &a, TileSmem<LIMC, R, TX, TY, NT,
   constexpr int DIR = KIND < 0 ? 4 : (GEOM ? 2 : 0) + KIND;
   s.ax = idir ? 0 : 1;
   edge_normal<GEOM>(a, idir, ci, cj, s);
-  edge_flux<R, FLUX, DIR, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2]), a.low_mach_fix, s, pn, f, &sb);
+  edge_flux<R, FLUX, DIR, DF>(gas_of<R>(a.gamma, a.gas[0], a.gas[1], a.gas[2], a.gas[3]), a.low_mach_fix, s, pn, f, &sb);
   return true;
 }
 
@@ -538,7 +538,9 @@ __device__ inline bool load_tile(Args &a, int i0, int j0, Sp &sp, int &err) {
 // right, top, left), volume and its reciprocal (FP64: the exact one of a power of
 // two, else 0; precision form: rounded).
 struct CellGeo {
-  double dxv, dyv, lb, lr, lt, ll, vol, inv_vol;
+  double dxv, dyv, lb, lr, lt, ll;
+  FastOps::Rcp<double> vol;
+  double inv_vol;
   bool pow2;
 };
 template <bool kExact, bool GEOM, class Args> __device__ inline CellGeo cell_geometry(Args &a, int gi, int gj) {
@@ -586,7 +588,8 @@ template <bool kExact, bool GEOM, class Args> __device__ inline CellGeo cell_geo
     const double inv_pow2 = __longlong_as_double((long long)((vb & 0x8000000000000000ull) | ((2046 - ve) << 52)));
     inv_vol = kExact ? (pow2 ? inv_pow2 : 0.0) : rcp64(vol);
   }
-  return CellGeo{dxv, dyv, lb, lr, lt, ll, vol, inv_vol, pow2};
+  const FastOps::Rcp<double> rv = kExact && !pow2 ? volume_rcp(vol) : FastOps::Rcp<double>{vol, 0.0};
+  return CellGeo{dxv, dyv, lb, lr, lt, ll, rv, inv_vol, pow2};
 }
 
 // d/dt of one variable of a cell from its edge fluxes (right, left, top, bottom).
