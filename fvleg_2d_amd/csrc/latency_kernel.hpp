@@ -151,7 +151,12 @@ __global__ __launch_bounds__(4 * TX * TY) void latency_kernel(StageArgs a) {
   // ---- 1. primitives of the tile + halo
   int err = 0;
   const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT>(a, i0, j0, sm.sp, err);
-  constexpr bool kFastScheme = fast_scheme<FLUX, LIMC, R>();
+  // The FastOps flux of the SLAU family and HLLC only: AUSM+, AUSMPW+ and Roe divide
+  // as IEEE does here.  Their FastOps forms shorten no chain (Sod 400 x 4 with AUSM+ 2 %
+  // slower) and take Roe to 159 registers, three workgroups a CU instead of five
+  // (301 x 243, rk(2,4), superbee: 6.39 -> 6.65 ms).
+  constexpr bool kFastFlux = slau_family<FLUX>() || FLUX == FLUX_HLLC;
+  constexpr bool kFastScheme = kExact && (kFastFlux || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
   if constexpr (kFastScheme) {
     const int vote = __all(in_range ? 1 : 0);
     if ((tid & 63) == 0) red.fast[tid >> 6] = vote;
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(4 * TX * TY) void latency_kernel(StageArgs a) {
     bool fast = a.fast_ops != 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) fast = fast && red.fast[w] != 0;
-    using DF = typename std::conditional<fast_ops_flux<FLUX>(), FastOps, IeeeOps>::type;
+    using DF = typename std::conditional<kFastFlux, FastOps, IeeeOps>::type;
     if (fast)
       latency_edges<FLUX, LIMC, R, TX, TY, FastOps, DF, GEOM, NT>(a, sm, i0, j0);
     else

@@ -242,7 +242,13 @@ struct FastOps {
 // |q| / c <= 2^42 < 2^52, so S_L - q_L and S_R - q_R keep at least half of c w
 // and m_L, m_R are nonzero within [2^-43, 2^88]; |S_L| >= 2^-75 where it
 // divides; S*, the star factors and the energy quotients lie within
-// [2^-400, 2^170].  No numerator of either is -0.
+// [2^-400, 2^170].  No numerator of either is -0.  AUSM+, AUSMPW+ and Roe on such
+// states: p / rho and the enthalpies lie within [2^-42, 2^47], the sound speeds and
+// the interface speeds built from them within [2^-140, 2^24] (AUSMPW+'s H_normal and
+// Roe's c2a, differences that can cancel, are checked on each edge), the Mach
+// numbers are 0 or within [2^-410, 2^170], AUSMPW+'s p_s is 0 (not divided by) or at
+// least 2^-130, and Roe's wave strengths are at most 2^200.  A numerator -0 (a normal
+// velocity, a wave strength) changes the sign of a zero there and no value.
 template <int LOG2B> __device__ inline bool fast_ops_cell(const Prim<double> &q) {
   static_assert(LOG2B >= 1 && LOG2B <= 60, "fast_ops_cell bound");
   constexpr double HI = (double)(1ull << LOG2B), LO = 1.0 / HI, VLO = 0x1p-150;
@@ -613,15 +619,16 @@ template <typename R> __device__ inline R pw_M_minus(R M) {
 
 // min(p_L / p_R, p_R / p_L).  FP64: of two positive finite pressures the smaller
 // over the larger, since rounding keeps both quotients on their side of 1.
-template <typename R> __device__ inline R pw_ratio(R p_L, R p_R) {
+template <typename R, class D = IeeeOps> __device__ inline R pw_ratio(R p_L, R p_R) {
   if constexpr (std::is_same<R, double>::value) {
     const R lo = fmin2(p_L, p_R), hi = fmax2(p_L, p_R);
+    if constexpr (std::is_same<D, FastOps>::value) return D::div(lo, hi);
     if (lo > R(0) && hi <= R(1.7976931348623157e308)) return lo / hi;
   }
   return fmin2((p_L / p_R), (p_R / p_L));
 }
 
-template <typename R, int DIR>
+template <typename R, int DIR, class D = IeeeOps>
 __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const EdgeState<R> &s, const PressNbr<R> &pn,
                                    R out[4]) {
   const R n_x = edge_nx<R, DIR>(s), n_y = edge_ny<R, DIR>(s);
@@ -631,10 +638,11 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
   R U_L = edge_ax0<R, DIR>(s) ? u_LHS : v_LHS, U_R = edge_ax0<R, DIR>(s) ? u_RHS : v_RHS;
   R V_L = edge_ax0<R, DIR>(s) ? v_LHS : u_LHS, V_R = edge_ax0<R, DIR>(s) ? v_RHS : u_RHS;
   const R gamma = gas.gamma;
-  R cs_L = sqrtr(gamma * p_L / rho_L);
-  R cs_R = sqrtr(gamma * p_R / rho_R);
-  R M_LHS = sqrtr(sq(u_LHS) + sq(v_LHS)) / cs_L;
-  R M_RHS = sqrtr(sq(u_RHS) + sq(v_RHS)) / cs_R;
+  const auto dr_L = D::rcp(rho_L), dr_R = D::rcp(rho_R);
+  R cs_L = D::sqrt_pos(D::div(gamma * p_L, dr_L));
+  R cs_R = D::sqrt_pos(D::div(gamma * p_R, dr_R));
+  R M_LHS = D::div(D::sqrt0(sq(u_LHS) + sq(v_LHS)), cs_L);
+  R M_RHS = D::div(D::sqrt0(sq(u_RHS) + sq(v_RHS)), cs_R);
   if (low_mach_fix && (absd(M_LHS) < LOW_MACH || absd(M_RHS) < LOW_MACH)) {
     R f_M = fmin2(R(1), fmax2(M_LHS, M_RHS));
     R ulf = R(0.5) * (u_LHS + u_RHS) + f_M * R(0.5) * (u_LHS - u_RHS);
@@ -644,19 +652,26 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
     u_LHS = ulf; u_RHS = urf; v_LHS = vlf; v_RHS = vrf;
   }
   R gg = gas.gg;
-  R H_L = gg * (p_L / rho_L) + R(0.5) * (sq(u_LHS) + sq(v_LHS));
-  R H_R = gg * (p_R / rho_R) + R(0.5) * (sq(u_RHS) + sq(v_RHS));
+  R H_L = gg * D::div(p_L, dr_L) + R(0.5) * (sq(u_LHS) + sq(v_LHS));
+  R H_R = gg * D::div(p_R, dr_R) + R(0.5) * (sq(u_RHS) + sq(v_RHS));
   R H_normal = fmin2(H_L - R(0.5) * sq(V_L), H_R - R(0.5) * sq(V_R));
-  R c_s = sqrtr(gas.cr2 * H_normal);
-  R c_half = (R(0.5) * (U_L + U_R) < R(0)) ? sq(c_s) / fmax2(absd(U_R), c_s) : sq(c_s) / fmax2(absd(U_L), c_s);
-  R M_L = U_L / c_half;
-  R M_R = U_R / c_half;
+  if constexpr (std::is_same<D, FastOps>::value) {
+    // a transverse speed so far above the sound speed that H_normal cancels (to
+    // below its last bits, zero or a negative): the IEEE operations
+    if (!(H_normal >= 0x1p-100)) return flux_ausmpw<R, DIR, IeeeOps>(gas, low_mach_fix, s, pn, out);
+  }
+  R c_s = D::sqrt_pos(gas.cr2 * H_normal);
+  R c_half = (R(0.5) * (U_L + U_R) < R(0)) ? D::div(sq(c_s), fmax2(absd(U_R), c_s))
+                                           : D::div(sq(c_s), fmax2(absd(U_L), c_s));
+  const auto dc = D::rcp(c_half);
+  R M_L = D::div(U_L, dc);
+  R M_R = D::div(U_R, dc);
   R M_L_plus = pw_M_plus(M_L);
   R M_R_minus = pw_M_minus(M_R);
   R P_R_minus = pw_P_minus(M_R);
   R P_L_plus = pw_P_plus(M_L);
   R p_s = p_L * P_L_plus + p_R * P_R_minus;
-  R mt = pw_ratio(p_L, p_R);
+  R mt = pw_ratio<R, D>(p_L, p_R);
   R w = R(1) - mt * mt * mt;
   // get_f neighbours (ausmpw_plus_solver.fypp:433-441): i-dir p1=(0,-1),(1,-1) p2=(0,+1),(1,+1);
   // j-dir p1=(i+1,j),(i+1,j+1) p2=(i-1,j),(i-1,j+1), i.e. transverse +1 then -1.
@@ -668,10 +683,11 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
     f_R = R(0);
   } else {
     R mn4 = fmin2(fmin2(fmin2(p1L, p1R), p2L), p2R);
-    R m1 = fmin2(R(1), mn4 / fmin2(p_L, p_R));
+    R m1 = fmin2(R(1), D::div(mn4, fmin2(p_L, p_R)));
     R min_term = sq(m1);
-    f_L = ((p_L / p_s) - R(1)) * min_term;
-    f_R = ((p_R / p_s) - R(1)) * min_term;
+    const auto dp_s = D::rcp(p_s);
+    f_L = (D::div(p_L, dp_s) - R(1)) * min_term;
+    f_R = (D::div(p_R, dp_s) - R(1)) * min_term;
   }
   R Mb_L, Mb_R;
   if (M_L_plus + M_R_minus < R(0)) {
@@ -700,39 +716,51 @@ template <typename R> __device__ inline R roe_f_h(R pL, R pR) {
   return (ratio < R(1)) ? R(0) : R(1);
 }
 
-template <typename R, int DIR>
+template <typename R, int DIR, class D = IeeeOps>
 __device__ inline void flux_roe(const Gas<R> &gas, const EdgeState<R> &s, const PressNbr<R> &pn, R out[4]) {
   const R nx = edge_nx<R, DIR>(s), ny = edge_ny<R, DIR>(s);
   R rl = absd(s.rL), ul = s.uL, vl = s.vL, pl = absd(s.pL);
   const R gamma = gas.gamma;
   R gg = gas.gg;
-  R hl = gg * (pl / rl) + R(0.5) * (sq(ul) + sq(vl));
+  const auto d_rl = D::rcp(rl);
+  R hl = gg * D::div(pl, d_rl) + R(0.5) * (sq(ul) + sq(vl));
   R rr = absd(s.rR), ur = s.uR, vr = s.vR, pr = absd(s.pR);
-  R hr = gg * (pr / rr) + R(0.5) * (sq(ur) + sq(vr));
-  R rav = sqrtr(rl * rr);
+  const auto d_rr = D::rcp(rr);
+  R hr = gg * D::div(pr, d_rr) + R(0.5) * (sq(ur) + sq(vr));
+  R rav = D::sqrt_pos(rl * rr);
   R gam1 = gamma - R(1);
-  R dd = rav / rl;
-  R dd1 = R(1) / (R(1) + dd);
+  R dd = D::div(rav, d_rl);
+  R dd1 = D::div(R(1), R(1) + dd);
   R uav = (ul + dd * ur) * dd1;
   R vav = (vl + dd * vr) * dd1;
   R hav = (hl + dd * hr) * dd1;
   R q2a = R(0.5) * (uav * uav + vav * vav);
   R c2a = gam1 * (hav - q2a);
-  R cav = sqrtr(c2a);
+  if constexpr (std::is_same<D, FastOps>::value) {
+    // a speed so far above the sound speed that c2a cancels: the IEEE operations
+    if (!(c2a >= 0x1p-100)) return flux_roe<R, DIR, IeeeOps>(gas, s, pn, out);
+  }
+  R cav = D::sqrt_pos(c2a);
   R uv = uav * nx + vav * ny;
   R du = (ur - ul) * nx + (vr - vl) * ny;
   R du_trans = -((ur - ul) * ny) + (vr - vl) * nx;
-  R cs_R = sqrtr(gamma * pr / rr);
-  R cs_L = sqrtr(gamma * pl / rl);
+  R cs_R = D::sqrt_pos(D::div(gamma * pr, d_rr));
+  R cs_L = D::sqrt_pos(D::div(gamma * pl, d_rl));
   R eabs1 = absd(fmin2(uv - cav, (ul * nx + vl * ny) - cs_L));
   R eabs2 = absd(uv);
   R eabs4 = absd(fmax2(uv + cav, (ur * nx + vr * ny) + cs_R));
   R h1 = rav * cav * du;
-  R h2 = eabs1 * (pr - pl - h1) / (R(2) * c2a);
-  R h3 = eabs2 * (rr - rl - (pr - pl) / c2a);
+  // a quotient by 2 c2a is half the one by c2a, exactly (FastOps: none is subnormal)
+  const auto dc2 = D::rcp(c2a);
+  auto over_2c2 = [&](R x) {
+    if constexpr (std::is_same<D, FastOps>::value) return R(0.5) * D::div(x, dc2);
+    else return x / (R(2) * c2a);
+  };
+  R h2 = over_2c2(eabs1 * (pr - pl - h1));
+  R h3 = eabs2 * (rr - rl - D::div(pr - pl, dc2));
   R h4 = eabs2 * rav;
-  R h5 = eabs4 * (pr - pl + h1) / (R(2) * c2a);
-  R psi = absd(cs_R - cs_L) / fmax2(cs_R, cs_L);
+  R h5 = over_2c2(eabs4 * (pr - pl + h1));
+  R psi = D::div(absd(cs_R - cs_L), fmax2(cs_R, cs_L));
   R FR0 = rr * uv, FR1 = rr * ur * uv + nx * pr, FR2 = rr * vr * uv + ny * pr, FR3 = rr * hr * uv;
   R FL0 = rl * uv, FL1 = rl * ul * uv + nx * pl, FL2 = rl * vl * uv + ny * pl, FL3 = rl * hl * uv;
   R rm0 = (h2 + h3 + h5);
@@ -765,7 +793,7 @@ __device__ inline void flux_roe(const Gas<R> &gas, const EdgeState<R> &s, const 
 
 // AUSM+ from interface_state (ausm_plus_solver.f90:499-643) with the AUSM+-u flags
 // (M_p = p_u = 0), beta = 1/8, alpha = 3/16, upwinded as in the commented solve (312-325).
-template <typename R, int DIR>
+template <typename R, int DIR, class D = IeeeOps>
 __device__ inline void flux_ausm_plus(const Gas<R> &gas, const EdgeState<R> &s, R out[4]) {
   const R n_x = edge_nx<R, DIR>(s), n_y = edge_ny<R, DIR>(s);
   const R beta = R(1) / R(8), alpha = R(3) / R(16);
@@ -776,15 +804,16 @@ __device__ inline void flux_ausm_plus(const Gas<R> &gas, const EdgeState<R> &s, 
   R vel_L = u_L * n_x + v_L * n_y;
   R vel_R = u_R * n_x + v_R * n_y;
   R gg = gas.gg;
-  R H_L = (p_L / rho_L) * gg + R(0.5) * (u_L * u_L + v_L * v_L);
-  R H_R = (p_R / rho_R) * gg + R(0.5) * (u_R * u_R + v_R * v_R);
-  R a_crit_L = sqrtr(gamma_factor * absd(H_L));
-  R a_crit_R = sqrtr(gamma_factor * absd(H_R));
-  R a_circ_L = sq(a_crit_L) / fmax2(a_crit_L, vel_L);
-  R a_circ_R = sq(a_crit_R) / fmax2(a_crit_R, -vel_R);
-  R a_half = fmin2(a_circ_L, a_circ_R);
-  R M_L = vel_L / a_half;
-  R M_R = vel_R / a_half;
+  R H_L = D::div(p_L, rho_L) * gg + R(0.5) * (u_L * u_L + v_L * v_L);
+  R H_R = D::div(p_R, rho_R) * gg + R(0.5) * (u_R * u_R + v_R * v_R);
+  R a_crit_L = D::sqrt_pos(gamma_factor * absd(H_L));
+  R a_crit_R = D::sqrt_pos(gamma_factor * absd(H_R));
+  R a_circ_L = D::div(sq(a_crit_L), D::max(a_crit_L, vel_L));
+  R a_circ_R = D::div(sq(a_crit_R), D::max(a_crit_R, -vel_R));
+  R a_half = D::min(a_circ_L, a_circ_R);
+  const auto da = D::rcp(a_half);
+  R M_L = D::div(vel_L, da);
+  R M_R = D::div(vel_R, da);
   R M2p_L = R(0.25) * sq(M_L + R(1)), M2m_L = -(R(0.25) * sq(M_L - R(1)));
   R M2p_R = R(0.25) * sq(M_R + R(1)), M2m_R = -(R(0.25) * sq(M_R - R(1)));
   R M_plus = (absd(M_L) >= R(1)) ? R(0.5) * (M_L + absd(M_L)) : M2p_L * (R(1) - R(16) * beta * M2m_L);
@@ -996,24 +1025,27 @@ template <int FLUX> constexpr bool needs_superbee_states() { return FLUX == FLUX
 template <typename R, int FLUX, int DIR, class D = IeeeOps>
 __device__ inline void edge_flux(const Gas<R> &gas, int low_mach_fix, const EdgeState<R> &s, const PressNbr<R> &pn,
                                  R out[4], const EdgeState<R> *sb = nullptr) {
-  if constexpr (FLUX == FLUX_AUSMPW_PLUS) flux_ausmpw<R, DIR>(gas, low_mach_fix, s, pn, out);
+  if constexpr (FLUX == FLUX_AUSMPW_PLUS) flux_ausmpw<R, DIR, D>(gas, low_mach_fix, s, pn, out);
   else if constexpr (FLUX == FLUX_M_AUSMPW_PLUS) flux_m_ausmpw<R, DIR>(gas, low_mach_fix, s, *sb, pn, out);
   else if constexpr (FLUX == FLUX_SLAU || FLUX == FLUX_SLAU2 || FLUX == FLUX_SD_SLAU || FLUX == FLUX_SD_SLAU2)
     flux_slau<R, FLUX, DIR, D>(gas, s, pn, out);
-  else if constexpr (FLUX == FLUX_ROE) flux_roe<R, DIR>(gas, s, pn, out);
-  else if constexpr (FLUX == FLUX_AUSM_PLUS) flux_ausm_plus<R, DIR>(gas, s, out);
+  else if constexpr (FLUX == FLUX_ROE) flux_roe<R, DIR, D>(gas, s, pn, out);
+  else if constexpr (FLUX == FLUX_AUSM_PLUS) flux_ausm_plus<R, DIR, D>(gas, s, out);
   else flux_hllc<R, DIR, D>(gas, s, out);
 }
 
-// FP64 fluxes with a FastOps path (the SLAU family and HLLC; every limiter has
+// FP64 fluxes with a FastOps path (every one but M-AUSMPW+; every limiter has
 // one), and the bound B of fast_ops_cell that keeps a scheme's operations in
-// range: 60 for TVD2 with the SLAU family, 20 otherwise.
-template <int FLUX> constexpr bool fast_ops_flux() {
-  return FLUX == FLUX_SLAU || FLUX == FLUX_SLAU2 || FLUX == FLUX_SD_SLAU || FLUX == FLUX_SD_SLAU2 ||
-         FLUX == FLUX_HLLC;
+// range: 60 for TVD2 with the SLAU family, 20 otherwise.  What it took off a stage
+// of 1024 x 987 cells on 32 x 8 tiles, van Leer / MLP5 (the range vote included):
+// AUSM+ 73.5 -> 67.0 / 119.6 -> 109.7 us, AUSMPW+ 88.0 -> 77.8 / 134.7 -> 121.8 us,
+// Roe 93.7 -> 80.0 / 139.0 -> 122.2 us.
+template <int FLUX> constexpr bool slau_family() {
+  return FLUX == FLUX_SLAU || FLUX == FLUX_SLAU2 || FLUX == FLUX_SD_SLAU || FLUX == FLUX_SD_SLAU2;
 }
+template <int FLUX> constexpr bool fast_ops_flux() { return FLUX != FLUX_M_AUSMPW_PLUS; }
 template <int FLUX, int LIMC> constexpr int fast_ops_bound() {
-  return (FLUX != FLUX_HLLC && fast_ops_flux<FLUX>() && LIMC != LIM_MLP3 && LIMC != LIM_MLP5) ? 60 : 20;
+  return (slau_family<FLUX>() && LIMC != LIM_MLP3 && LIMC != LIM_MLP5) ? 60 : 20;
 }
 
 template <int FLUX> constexpr bool needs_pressure_nbrs() {

@@ -474,7 +474,7 @@ __device__ inline void edge_pass(Args &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &
 // cells through the boundary map.  Adds 1 to err where a checked cell holds a NaN;
 // returns whether every cell this thread loaded keeps the FastOps operations of
 // the reconstruction and of the flux (where it has a FastOps path) in range
-// (fast_ops_cell).  TVD2 under a flux without one divides too little for the
+// (fast_ops_cell).  TVD2 under M-AUSMPW+, which has none, divides too little for the
 // range vote to pay.
 template <int FLUX, int LIMC, typename R> constexpr bool fast_scheme() {
   return !std::is_same<R, f32x>::value && (fast_ops_flux<FLUX>() || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);

@@ -82,3 +82,19 @@ def test_pressure_ratios(oracle, flux):
             got = s.edge_fluxes(edges, p)
     for g, w in zip(got, want):
         assert np.array_equal(g, w, equal_nan=True)
+
+
+# in-range cells (speeds below 2^20, densities and pressures in [2^-20, 2^20]) whose sound speed is lost beside
+# the flow speed: AUSMPW+'s normal enthalpy and Roe's c^2 cancel, to zero or a negative number on some edges
+@pytest.mark.parametrize("tile", [-1, 0])
+@pytest.mark.parametrize("limiter", ["minmod", "van_leer", "MLP5"])
+@pytest.mark.parametrize("flux", ["Roe", "AUSMPW+", "AUSM+", "HLLC"])
+def test_cancelled_sound_speeds(oracle, flux, limiter, tile):
+    rng = np.random.default_rng(6)
+    shape = (NI, NJ)
+    prims = [rng.uniform(1e5, 9e5, shape), rng.choice([0.0, 3.0, 9e5, -9e5], shape) * rng.choice([1.0, 1 + 1e-9], shape),
+             rng.choice([1.0, 9e5, 9.1e5, -8e5], shape), rng.uniform(1e-6, 3e-6, shape)]
+    with np.errstate(all="ignore"):
+        got, want = both_residuals(oracle, flux, limiter, [np.asfortranarray(a) for a in prims], tile=tile)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w, equal_nan=True)
