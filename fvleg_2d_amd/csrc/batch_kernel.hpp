@@ -35,8 +35,9 @@ struct BatchSolveRef {
 struct BatchStageArgs {
   const StageArgs *args;   // per solve, this stage
   const int *variant;      // per solve: flux * LIM_COUNT + limiter
-  const BatchItem *items;  // work list, grouped by variant and solve
-  const int *count;        // number of live entries of items (device-resident: graph replays see updates)
+  const BatchItem *items;  // work list (build_work_list)
+  const int *slices;       // its kNumXcd slices: slice x is entries slices[x] to slices[x + 1] (device-resident:
+                           // graph replays see updates)
   int *cursor;             // kNumXcd work cursors of this stage, kCursorStride apart: zero at launch, reset by
                            // the finalize kernel
 };
@@ -68,7 +69,9 @@ template <typename T> __device__ inline ConstPtr<T> table(const T *p) { return (
 
 // Waves per SIMD the LDS footprint allows (at most 4): the register budget is
 // capped to match, since the forty variants merged in one body would
-// otherwise claim far more registers than any single variant needs.
+// otherwise claim far more registers than any single variant needs.  (More waves
+// of the precision form, whose LDS would hold eight, spill: 32 solves of side 64 to
+// 256 take 46 us a stage with four, 52 us with six or eight.)
 template <typename R, int TX, int TY> constexpr int batch_waves_per_simd() {
   constexpr size_t lds = batch_smem_bytes<R, TX, TY>() + sizeof(RedSmem);
   constexpr int fit = (int)((160 * 1024) / lds);
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(kThreads, (batch_waves_per_simd<R, TX, TY>())) void
   __shared__ __attribute__((aligned(16))) char smem[batch_smem_bytes<R, TX, TY>()];
   __shared__ RedSmem red;
   __shared__ int s_item;
-  // The work list is cut into kNumXcd contiguous slices.  Workgroups of XCD x
+  // The work list is cut into kNumXcd slices.  Workgroups of XCD x
   // take items of slice x (neighbouring tiles stay in one L2), the first of them
   // by position and the others through the slice's cursor, then help the other
   // slices: items differ in cost by variant, so a static split would leave XCDs
@@ -88,9 +91,8 @@ __global__ __launch_bounds__(kThreads, (batch_waves_per_simd<R, TX, TY>())) void
   // workgroup starts on the one it has and looks at the answer after it, so that
   // the atomic's round trip lies under the tile's work; and it looks at another
   // slice's cursor before it adds to it, so that drained slices cost a load.
-  const int nitems = *b.count;
   const int x0 = blockIdx.x % kNumXcd, nwg = gridDim.x / kNumXcd;
-  auto slice = [&](int x) { return (int)(((long long)nitems * x) / kNumXcd); };
+  auto slice = [&](int x) { return table(b.slices)[x]; };
   auto cursor = [&](int x) { return b.cursor + x * kCursorStride; };
   int x = x0, helped = 0, base = slice(x0), taken = (int)blockIdx.x / kNumXcd;  // of thread 0: item base + taken
   while (true) {

@@ -21,8 +21,8 @@ struct BatchEngine {
   std::vector<int> pin;
   size_t pass_off = 0;
   std::vector<BatchItem> live_items;  // host copy of the current work list
-  std::vector<int> order;             // solves ordered by kernel variant
-  int live_solves = 0, live_count = 0;
+  int live_slices[kNumXcd + 1] = {};
+  int live_solves = 0;
   int precision = 0, tile = 0, nstages = 0, nitems = 0, grid = 0;
   BatchLauncher launcher = nullptr;
   hipGraph_t graph = nullptr;
@@ -32,6 +32,7 @@ struct BatchEngine {
   void release();
   int upload_args();
   int launch_step(bool first);
+  void list_items(const std::vector<LoopState> *H);
   int compact(const std::vector<LoopState> &H);
   int set_pressure_input(int k, const double *time, const double *pressure, const double *density, int n);
   int run(const double *max_time, const double *contour_dt, long long max_iterations, int use_graph,

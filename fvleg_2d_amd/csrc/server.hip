@@ -99,7 +99,7 @@ struct cato_server {
          cursor_off = 0, pass_off = 0;
   int npin = 0;  // resident solves with a +x pressure input (their column passes: [stage slot][npin])
   std::vector<BatchItem> items;  // host copy of the work list (kept until the next tick)
-  int item_count = 0;
+  int slices[kNumXcd + 1] = {};
   int max_items = 0, resident_items = 0;
   Arena arena;
   std::vector<Request> reqs;
@@ -166,7 +166,6 @@ int server_upload(cato_server *S, int &nitems, std::vector<int> &active_ids) {
   std::vector<int> variant(n, 0);
   std::vector<BatchSolveRef> refs;
   std::vector<BatchItem> &items = S->items;
-  items.clear();
   active_ids.clear();
   for (int k = 0; k < n; ++k) {
     Slot &sl = S->slots[k];
@@ -190,20 +189,17 @@ int server_upload(cato_server *S, int &nitems, std::vector<int> &active_ids) {
     refs.push_back(BatchSolveRef{sv.block_min, sv.block_err, sv.loop, nt, 0});
     active_ids.push_back(k);
   }
-  // work list grouped by kernel variant (instruction-cache locality per XCD slice)
-  std::vector<int> order(active_ids);
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return variant[x] < variant[y]; });
-  for (int k : order) {
+  std::vector<BatchShare> shares;
+  for (int k : active_ids) {
     const Solve &sv = *S->slots[k].s;
-    int nt = sv.tiles_x * sv.tiles_y;
-    if (nt >= kBigTiles) {
+    const int nt = sv.tiles_x * sv.tiles_y;
+    if (nt >= kBigTiles)
       S->big.push_back(k);
-      continue;
-    }
-    for (int t = 0; t < nt; ++t) items.push_back({k, t});
+    else
+      shares.push_back({k, nt, variant[k]});
   }
+  build_work_list(std::move(shares), items, S->slices);
   nitems = (int)items.size();
-  S->item_count = nitems;
   if (nitems > S->max_items) return fail(CATO_ERR_INVALID, "internal: server work list overflow");
   // +x pressure-input passes of the resident solves that have one, before every stage
   std::vector<int> pin;
@@ -235,7 +231,7 @@ int server_upload(cato_server *S, int &nitems, std::vector<int> &active_ids) {
                                                items.size() * sizeof(BatchItem), hipMemcpyHostToDevice, st),
                                 "items")))
     return rc;
-  if ((rc = hip_check(hipMemcpyAsync(S->table_mem + S->count_off, &S->item_count, sizeof(int),
+  if ((rc = hip_check(hipMemcpyAsync(S->table_mem + S->count_off, S->slices, sizeof(S->slices),
                                      hipMemcpyHostToDevice, st), "count")))
     return rc;
   // pageable host vectors: wait before they go out of scope (tab is kept for the big solves' launches)
@@ -367,7 +363,7 @@ int enqueue_tick(cato_server *S, bool first_fresh, int grid, int resident) {
         b.args = args + (size_t)slot * n;
         b.variant = reinterpret_cast<const int *>(S->table_mem + S->variant_off);
         b.items = reinterpret_cast<const BatchItem *>(S->table_mem + S->items_off);
-        b.count = reinterpret_cast<const int *>(S->table_mem + S->count_off);
+        b.slices = reinterpret_cast<const int *>(S->table_mem + S->count_off);
         b.cursor = reinterpret_cast<int *>(S->table_mem + S->cursor_off) + (size_t)s * kCursorInts;
         S->launcher(dim3((unsigned)grid), S->stream, b);
       }
@@ -429,7 +425,7 @@ int cato_server_create(double hbm_budget_bytes, int max_slots, int precision, in
   int cus = (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
                 ? prop.multiProcessorCount
                 : 256;
-  S->grid = 4 * cus;
+  S->grid = batch_wgs_per_cu(precision, S->tile) * cus;
   *out = S;
   return CATO_OK;
 }
