@@ -254,17 +254,39 @@ static int validate_config(const cato_config &c) {
   return CATO_OK;
 }
 
-// The library's choice of tile: the latency layout up to five of its tiles per CU, 32 x 8 above.  Measured
-// with five schemes in both precisions, us per SSP-RK3 step with 32 x 8 tiles / in the latency layout:
-// 64^2 35-51 / 21-25 (FP64) and 26-35 / 15-17 (FP32 flux); 256^2 35-52 / 32-43 and 25-35 / 21-27;
-// 272^2 (1156 tiles) 40-64 / 36-49 and 28-40 / 23-30; FP64 288^2 (1296 tiles) 40-64 / 42-58.
-constexpr int kLatencyTiles = 5 * 256;
+// The library's choice of tile for a solve with launches of its own.
+//
+// Up to five 8 x 8 tiles per CU: the latency layout.  Measured with five schemes in both precisions, us per
+// SSP-RK3 step with 32 x 8 tiles / in the latency layout: 64^2 35-51 / 21-25 (FP64) and 26-35 / 15-17 (FP32
+// flux); 256^2 35-52 / 32-43 and 25-35 / 21-27; 272^2 (1156 tiles) 40-64 / 36-49 and 28-40 / 23-30; FP64
+// 288^2 (1296 tiles) 40-64 / 42-58.
+//
+// Above, 32 x 16 where its fewer edges and halo cells per cell pay: with at least four such tiles per CU (with
+// fewer, the last round of tiles is too empty: 640^2, 3.1 per CU, is 3 to 8 % slower), in FP64 unless the
+// scheme's registers take its occupancy (Roe, AUSMPW+ and M-AUSMPW+ with MLP5: 2 to 4 % slower), and in the
+// precision form with MLP5 or from 1.5 M cells on.  Elsewhere 16 x 16.  us a stage with 16 x 16 / 32 x 16
+// tiles (32 x 8): FP64 1024^2 HLLC + MLP5 111.4 / 106.9 (112.6), SLAU2 + MLP3 92.0 / 88.4 (92.9), Roe + van
+// Leer 84.4 / 85.9 (82.7), 2048^2 AUSMPW+ + MLP5 421 / 434 (424), SLAU + van Leer 240.6 / 241.4 (240.2);
+// FP32 flux 1024^2 HLLC + MLP5 56.2 / 55.0 (58.2), SLAU + van Leer 36.3 / 37.3 (37.6), 2048^2 133.6 / 129.2
+// (129.9).
+constexpr int kCus = 256;
+constexpr int kLatencyTiles = 5 * kCus;
 
 static int default_tile(const cato_config &c, int ni, int nj, bool single) {
   if (c.tile >= 0) return c.tile;
-  const TileShape t = kTiles[kLatencyTile];
-  const long long tiles = (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
-  return single && tiles <= kLatencyTiles ? kLatencyTile : 0;
+  if (!single) return 0;
+  auto count = [&](int tile) {
+    const TileShape t = kTiles[tile];
+    return (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
+  };
+  if (count(kLatencyTile) <= kLatencyTiles) return kLatencyTile;
+  const bool mlp5 = c.limiter == LIM_MLP5;
+  bool wide;
+  if (c.precision == CATO_PRECISION_FP64)
+    wide = c.flux != FLUX_ROE && !(mlp5 && (c.flux == FLUX_AUSMPW_PLUS || c.flux == FLUX_M_AUSMPW_PLUS));
+  else
+    wide = mlp5 || (long long)ni * nj >= 1500000;
+  return wide && count(1) >= 4 * kCus ? 1 : 2;
 }
 
 int Solve::init(const cato_config &c, const cato_geom &g, bool single) {
@@ -296,10 +318,11 @@ int Solve::init(const cato_config &c, const cato_geom &g, bool single) {
 
 size_t Solve::field_elems() const { return (size_t)pitch * nj; }
 
-// Tiles whose partials lie within device_bytes(): the solve's own, except that those of the latency layout
-// lie in its tail and the 32 x 8 tiles it stands for count here.
+// Tiles whose partials device_bytes() counts: the solve's own, or where the library chose them the 32 x 8
+// ones (quad cells: 16 x 16) that every single solve once had, so that a footprint does not depend on the
+// choice.  A single solve's partials lie in its tail.
 size_t Solve::counted_tiles() const {
-  const TileShape t = kTiles[tile == kLatencyTile ? 0 : tile];
+  const TileShape t = kTiles[cfg.tile >= 0 && !geo.quad ? tile : geo.quad ? kQuadTile : 0];
   return (size_t)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
 }
 
@@ -341,7 +364,7 @@ void Solve::bind(char *base) {
 }
 
 // What a single solve keeps after its device_bytes(): the second copies of the loop state and the sanity
-// flags (StageArgs::fold_n), and the partials of the latency layout's tiles, more than a batched solve's.
+// flags (StageArgs::fold_n), and the partials of its tiles.
 size_t Solve::tail_bytes() const {
   return 256 + sizeof(LoopState) + (size_t)tiles_x * tiles_y * (sizeof(double) + 2 * sizeof(int));
 }
