@@ -150,7 +150,7 @@ __global__ __launch_bounds__(4 * TX * TY) void latency_kernel(StageArgs a) {
 
   // ---- 1. primitives of the tile + halo
   int err = 0;
-  const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT>(a, i0, j0, sm.sp, err);
+  const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT, false>(a, i0, j0, sm.sp, err);
   // The FastOps flux of the SLAU family and HLLC only: AUSM+, AUSMPW+ and Roe divide
   // as IEEE does here.  Their FastOps forms shorten no chain (Sod 400 x 4 with AUSM+ 2 %
   // slower) and take Roe to 159 registers, three workgroups a CU instead of five

@@ -479,7 +479,8 @@ __device__ inline void edge_pass(Args &a, TileSmem<LIMC, R, TX, TY, NT, SPLIT> &
 template <int FLUX, int LIMC, typename R> constexpr bool fast_scheme() {
   return !std::is_same<R, f32x>::value && (fast_ops_flux<FLUX>() || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
 }
-template <int FLUX, int LIMC, typename R, int TX, int TY, int NT, class Args, class Sp>
+// AHEAD: ask for every cell of the thread before using the first.
+template <int FLUX, int LIMC, typename R, int TX, int TY, int NT, bool AHEAD, class Args, class Sp>
 __device__ inline bool load_tile(Args &a, int i0, int j0, Sp &sp, int &err) {
   constexpr int H = halo_of<LIMC>();
   constexpr int RX = TX + 2 * H, RY = TY + 2 * H;
@@ -495,23 +496,31 @@ __device__ inline bool load_tile(Args &a, int i0, int j0, Sp &sp, int &err) {
   if (inner) {
     const bool check = recover || a.check_input;
     const size_t base = (size_t)(j0 - H - 1) * a.pitch + (size_t)(i0 - H - 1);
-    for (int idx = tid; idx < RX * RY; idx += NT) {
-      int ly = idx / RX, lx = idx - ly * RX;
-      const size_t off = base + (size_t)ly * a.pitch + (size_t)lx;
-      Prim<double> pr;
-      if (recover) {
-        double cs;
-        const Prim<double> U = load4(a.uk[0], off, a.fstride);
-        pr = cons_to_prim_fast(U.rho, U.u, U.v, U.p, a.gamma, a.gamma - 1.0, 0, &cs);
-      } else {
-        pr = load4(a.prim[0], off, a.fstride);
+    constexpr int K = AHEAD ? (RX * RY + NT - 1) / NT : 1;
+    const double *set = recover ? a.uk[0] : a.prim[0];
+    for (int first = tid; first < RX * RY; first += K * NT) {
+      Prim<double> q[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int idx = first + k * NT, ly = idx / RX, lx = idx - ly * RX;
+        if (K == 1 || idx < RX * RY) q[k] = load4(set, base + (size_t)ly * a.pitch + (size_t)lx, a.fstride);
       }
-      if (check && (pr.rho != pr.rho || pr.u != pr.u || pr.v != pr.v || pr.p != pr.p)) err |= 1;
-      if constexpr (kFastScheme) in_range = in_range && fast_ops_cell<fast_ops_bound<FLUX, LIMC>()>(pr);
-      sp[0][ly][lx] = (R)pr.rho;
-      sp[1][ly][lx] = (R)pr.u;
-      sp[2][ly][lx] = (R)pr.v;
-      sp[3][ly][lx] = (R)pr.p;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int idx = first + k * NT, ly = idx / RX, lx = idx - ly * RX;
+        if (K > 1 && idx >= RX * RY) break;
+        Prim<double> pr = q[k];
+        if (recover) {
+          double cs;
+          pr = cons_to_prim_fast(pr.rho, pr.u, pr.v, pr.p, a.gamma, a.gamma - 1.0, 0, &cs);
+        }
+        if (check && (pr.rho != pr.rho || pr.u != pr.u || pr.v != pr.v || pr.p != pr.p)) err |= 1;
+        if constexpr (kFastScheme) in_range = in_range && fast_ops_cell<fast_ops_bound<FLUX, LIMC>()>(pr);
+        sp[0][ly][lx] = (R)pr.rho;
+        sp[1][ly][lx] = (R)pr.u;
+        sp[2][ly][lx] = (R)pr.v;
+        sp[3][ly][lx] = (R)pr.p;
+      }
     }
   } else {
     for (int idx = tid; idx < RX * RY; idx += NT) {
@@ -701,8 +710,18 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
   int err = 0;
 
   // ---- 1. primitives of the tile + halo ---------------------------------
+  // A wave that loads its tile issues before waves of other workgroups that are at
+  // their edges: its few instructions start a wait of microseconds that those
+  // waves' arithmetic then covers (KH 2048^2 FP64 245 -> 236 us, Riemann 1024^2 HLLC +
+  // MLP5 104 -> 99 us, precision form 1 %; the other way round it was 1 % slower).
+  // The precision form and MLP ask for all their cells at once: one memory latency
+  // for the tile instead of one per round of the workgroup over its cells (1 to 2 %
+  // of a stage; FP64 TVD2 is 2 % slower so, and the batched kernel spills).
   constexpr bool kFastScheme = fast_scheme<FLUX, LIMC, R>();
-  const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT>(a, i0, j0, sm.sp, err);
+  constexpr bool kAhead = !OUTFLOW_COL && (!kExact || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
+  __builtin_amdgcn_s_setprio(3);
+  const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT, kAhead>(a, i0, j0, sm.sp, err);
+  __builtin_amdgcn_s_setprio(0);
   if constexpr (kFastScheme) {
     const int vote = __all(in_range ? 1 : 0);
     if ((tid & 63) == 0) red.fast[tid >> 6] = vote;
