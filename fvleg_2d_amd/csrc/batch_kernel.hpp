@@ -142,34 +142,10 @@ __global__ __launch_bounds__(kThreads, (batch_waves_per_simd<R, TX, TY>())) void
 // zeroes the stage work cursors for the next step (all stages have finished).
 static __global__ __launch_bounds__(kThreads) void batch_finalize_kernel(const BatchSolveRef *refs, int mode,
                                                                        int *cursors, int ncursors) {
-  __shared__ double sm[kThreads / 64];
-  __shared__ int se[kThreads / 64];
   if (blockIdx.x == 0)
     for (int k = threadIdx.x; k < ncursors; k += kThreads) cursors[k] = 0;
-  const BatchSolveRef r = refs[blockIdx.x];
-  LoopState *L = r.loop;
-  if (mode == 2 && L->done) return;
-  double m = __builtin_inf();
-  int e = 0;
-  for (int k = threadIdx.x; k < r.ntiles; k += kThreads) {
-    double v = r.block_min[k];
-    m = (v < m) ? v : m;
-    e |= r.block_err[k];
-    r.block_err[k] = 0;
-  }
-  m = wave_min(m);
-  e = wave_or(e);
-  if ((threadIdx.x & 63) == 0) {
-    sm[threadIdx.x >> 6] = m;
-    se[threadIdx.x >> 6] = e;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int k = 0; k < kThreads / 64; ++k) {
-    m = (sm[k] < m) ? sm[k] : m;
-    e |= se[k];
-  }
-  loop_update(L, m, e, mode);
+  auto &r = table(refs)[blockIdx.x];
+  close_step<kThreads, 4>(r.ntiles, r.block_min, r.block_err, nullptr, r.loop, mode);
 }
 
 }  // namespace cato

@@ -262,8 +262,8 @@ int BatchEngine::run(const double *max_time, const double *contour_dt, long long
     for (int v = 0; v < 4; ++v) a[v] = sv.P[0][v];  // primitives of U^n
     hipLaunchKernelGGL(k_cfl_partial, dim3((unsigned)nb), dim3(kThreads), 0, stream, g, 1, a[0],
                        a[1], a[2], a[3], sv.block_min, sv.block_err);
-    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, stream, nb, sv.block_min, sv.block_err, sv.result,
-                       sv.loop, 1, ConvOut{});
+    hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, stream, nb, sv.block_min, sv.block_err, sv.result,
+                       sv.loop, 1);
     BCK(hipGetLastError());
   }
   // first step eagerly (its first stage reads the caller's primitives)

@@ -899,9 +899,13 @@ int launch_reduce(cato_ctx *c, int mode, bool with_conv) {
   int nb = s.tiles_x * s.tiles_y;
   return timed(c, false, [&] {
     // the convergence sums belong to a step (modes 0 and 2 after stages), not to a CFL pass
-    ConvOut cv = with_conv ? s.conv_out() : ConvOut{};
-    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, c->stream, nb, s.block_min, s.block_err, s.result,
-                       s.loop, mode, cv);
+    const ConvOut cv = with_conv ? s.conv_out() : ConvOut{};
+    if (cv.sums)
+      hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, c->stream, nb, s.block_min, s.block_err, s.result,
+                         s.loop, mode, cv);
+    else
+      hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, c->stream, nb, (const double *)s.block_min, s.block_err,
+                         s.result, s.loop, mode);
   });
 }
 
@@ -1208,8 +1212,8 @@ int cato_compute_dt_noalloc(cato_ctx *c, const double *rho, const double *u, con
   hipLaunchKernelGGL(k_cfl_partial, dim3((unsigned)nb), dim3(kThreads), 0, c->stream, g, 1, rho + off, u + off,
                      v + off, p + off, bmin, berr);
   HIPCK(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, c->stream, nb, bmin, berr, res, (LoopState *)nullptr,
-                     0, ConvOut{});
+  hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, c->stream, nb, (const double *)bmin, berr, res,
+                     (LoopState *)nullptr, 0);
   HIPCK(hipGetLastError());
   return hip_check(hipMemcpyAsync(dt_device, res, sizeof(double), hipMemcpyDeviceToDevice, c->stream),
                    "compute_dt_noalloc");

@@ -356,8 +356,8 @@ int cato_split_compute_dt(cato_split *S, double *dt) {
     const int nb = w.tiles_x * w.tiles_y;
     hipLaunchKernelGGL(k_cfl_partial, dim3((unsigned)nb), dim3(kThreads), 0, S->stream, w.fgeom(), 1, w.P[0][0],
                        w.P[0][1], w.P[0][2], w.P[0][3], w.block_min, w.block_err);
-    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, S->stream, nb, w.block_min, w.block_err, w.result,
-                       (LoopState *)nullptr, 0, ConvOut{});
+    hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, S->stream, nb, w.block_min, w.block_err, w.result,
+                       (LoopState *)nullptr, 0);
     SPCK(hipGetLastError());
     SPCK(hipMemcpyAsync(&r[(size_t)2 * s], w.result, 2 * sizeof(double), hipMemcpyDeviceToHost, S->stream));
   }
@@ -390,8 +390,8 @@ int cato_split_step(cato_split *S, double dt, int *error_code) {
   std::vector<double> r((size_t)2 * S->n);
   for (int s = 0; s < S->n; ++s) {
     Solve &w = S->sub[s];
-    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, S->stream, w.tiles_x * w.tiles_y, w.block_min,
-                       w.block_err, w.result, (LoopState *)nullptr, 0, ConvOut{});
+    hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, S->stream, w.tiles_x * w.tiles_y, w.block_min,
+                       w.block_err, w.result, (LoopState *)nullptr, 0);
     SPCK(hipGetLastError());
     SPCK(hipMemcpyAsync(&r[(size_t)2 * s], w.result, 2 * sizeof(double), hipMemcpyDeviceToHost, S->stream));
     w.prims_valid = false;
