@@ -129,8 +129,8 @@ int cato_tile_shape(int tile, int *tile_x, int *tile_y);
  * allocates the device-resident state.  Rectilinear grids keep separable 1D
  * geometry; any other quadrilateral grid keeps per-cell volumes, edge lengths,
  * min_dx / min_dy and edge normals (the flux path of flux_solver.f90:254-367,
- * 398-422 reads them) and runs the 16 x 16 tile.  A non-positive cell volume is
- * CATO_ERR_INVALID. */
+ * 398-422 reads them) and runs the 16 x 16 tile, or the library's layout for
+ * small grids.  A non-positive cell volume is CATO_ERR_INVALID. */
 int cato_ctx_create(const cato_config *cfg, const cato_geom *geom, cato_ctx **out);
 int cato_ctx_destroy(cato_ctx *ctx);
 
