@@ -259,7 +259,12 @@ static int validate_config(const cato_config &c) {
 // Up to five 8 x 8 tiles per CU: the latency layout.  Measured with five schemes in both precisions, us per
 // SSP-RK3 step with 32 x 8 tiles / in the latency layout: 64^2 35-51 / 21-25 (FP64) and 26-35 / 15-17 (FP32
 // flux); 256^2 35-52 / 32-43 and 25-35 / 21-27; 272^2 (1156 tiles) 40-64 / 36-49 and 28-40 / 23-30; FP64
-// 288^2 (1296 tiles) 40-64 / 42-58.
+// 288^2 (1296 tiles) 40-64 / 42-58.  Four per CU in FP64 with TVD2 under the SLAU family, Roe and M-AUSMPW+: more
+// than 96 registers leave a CU four of their workgroups, and a second round costs more than it saves.  16 x 16
+// tiles / latency layout at 254^2 (1024 tiles) and 270^2 (1156): Roe + superbee 36.1 / 37.7 and 43.6 / 47.9 us,
+// SLAU2 + minmod 32.8 / 32.2 and 38.4 / 41.4, SD-SLAU + superbee 34.5 / 34.1 and 41.5 / 44.0, M-AUSMPW+ + minmod
+// 44.1 / 43.9 and 52.2 / 54.7; where it stays (MLP, the other fluxes), SLAU2 + MLP3 50.4 / 47.0, Roe + MLP5
+// 62.4 / 57.3, HLLC + minmod 39.3 / 37.1.
 //
 // Above, 32 x 16 where its fewer edges and halo cells per cell pay: with at least four such tiles per CU (with
 // fewer, the last round of tiles is too empty: 640^2, 3.1 per CU, is 3 to 8 % slower), in FP64 unless the
@@ -279,8 +284,10 @@ static int default_tile(const cato_config &c, int ni, int nj, bool single) {
     const TileShape t = kTiles[tile];
     return (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
   };
-  if (count(kLatencyTile) <= kLatencyTiles) return kLatencyTile;
   const bool mlp5 = c.limiter == LIM_MLP5;
+  const bool four = c.precision == CATO_PRECISION_FP64 && !mlp5 && c.limiter != LIM_MLP3 &&
+                    c.flux != FLUX_HLLC && c.flux != FLUX_AUSM_PLUS && c.flux != FLUX_AUSMPW_PLUS;
+  if (count(kLatencyTile) <= (four ? 4 * kCus : kLatencyTiles)) return kLatencyTile;
   bool wide;
   if (c.precision == CATO_PRECISION_FP64)
     wide = c.flux != FLUX_ROE && !(mlp5 && (c.flux == FLUX_AUSMPW_PLUS || c.flux == FLUX_M_AUSMPW_PLUS));
