@@ -15,7 +15,8 @@ namespace cato {
 // 32 solves of side 64 to 256, whose waves waited for 75 % of their time.  That
 // batch took 43.7 ms for 64 steps (168 us a stage) and takes 31.9 ms with this
 // line, fewer atomics (batch_stage_kernel) and scalar arguments (table); 8 served
-// requests of side 128 to 384 took 40.4 ms and take 23.6 ms.
+// requests of side 128 to 384 took 40.4 ms and take 23.6 ms.  (25.9 and 23.4 ms now,
+// with the order of build_work_list and the loads ahead of stage_tile's barrier.)
 constexpr int kCursorStride = 32;
 constexpr int kCursorInts = kNumXcd * kCursorStride;  // per stage
 

@@ -270,10 +270,10 @@ static int validate_config(const cato_config &c) {
 // fewer, the last round of tiles is too empty: 640^2, 3.1 per CU, is 3 to 8 % slower), in FP64 unless the
 // scheme's registers take its occupancy (Roe, AUSMPW+ and M-AUSMPW+ with MLP5: 2 to 4 % slower), and in the
 // precision form with MLP5 or from 1.5 M cells on.  Elsewhere 16 x 16.  us a stage with 16 x 16 / 32 x 16
-// tiles (32 x 8): FP64 1024^2 HLLC + MLP5 111.4 / 106.9 (112.6), SLAU2 + MLP3 92.0 / 88.4 (92.9), Roe + van
-// Leer 84.4 / 85.9 (82.7), 2048^2 AUSMPW+ + MLP5 421 / 434 (424), SLAU + van Leer 240.6 / 241.4 (240.2);
-// FP32 flux 1024^2 HLLC + MLP5 56.2 / 55.0 (58.2), SLAU + van Leer 36.3 / 37.3 (37.6), 2048^2 133.6 / 129.2
-// (129.9).
+// tiles (32 x 8): FP64 1024^2 HLLC + MLP5 108.4 / 103.9 (111.7), Roe + superbee 73.7 / 76.9 (76.2), 2048^2 Roe +
+// superbee 257.8 / 269.1 (253.2), SLAU + van Leer 231.7 / 228.5 (231.0), AUSMPW+ + MLP5 (older kernels) 421 / 434
+// (424); FP32 flux 1024^2 HLLC + MLP5 55.0 / 54.2 (57.4), SLAU + van Leer 34.3 / 34.5 (34.6), 2048^2 125.2 / 119.2
+// (125.9).
 constexpr int kCus = 256;
 constexpr int kLatencyTiles = 5 * kCus;
 
