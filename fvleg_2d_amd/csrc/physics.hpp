@@ -1071,16 +1071,23 @@ __device__ inline void scaled_pair(double a, double b, double m, double &qa, dou
   qb = a_big ? q : copysignr(1.0, b);
 }
 
-// d / vol for a cell volume within [2^-400, 2^400] whose reciprocal the cell's four
-// variables share; |d| over 2^600, inf and NaN, and other volumes take the IEEE
-// division.  (A d below 2^-969 may lose its last bits: a rate that no sum keeps.)
+// d / vol for a cell volume (positive) within [2^-400, 2^400] whose reciprocal the
+// cell's four variables share; |d| over 2^600, inf and NaN, and other volumes take the
+// IEEE division.  A nonzero d is above 2^-101: divergence() flushes each of its two
+// balances below 1e-14 > 2^-47, so that their sum is 0 or at least 2^-53 of one.  The
+// remainder is formed with the opposite sign, and taken back so, because d = -fl is -0
+// wherever nothing flows: q = -0 then stays -0, as in the IEEE division, where the
+// other sign's +0 remainder turns it into +0.
 __device__ inline double over_volume(double d, const FastOps::Rcp<double> &vol) {
-  if (vol.y != 0.0 && absd(d) <= 0x1p600) return FastOps::div(d, vol);
+  if (vol.y != 0.0 && absd(d) <= 0x1p600) {
+    const double q = d * vol.y;
+    const double e = __builtin_fma(vol.b, q, -d);
+    return __builtin_fma(-e, vol.y, q);
+  }
   return d / vol.b;
 }
 __device__ inline FastOps::Rcp<double> volume_rcp(double vol) {
-  const double av = absd(vol);
-  return FastOps::Rcp<double>{vol, (av >= 0x1p-400 && av <= 0x1p400) ? FastOps::rcp(vol).y : 0.0};
+  return FastOps::Rcp<double>{vol, (vol >= 0x1p-400 && vol <= 0x1p400) ? FastOps::rcp(vol).y : 0.0};
 }
 
 // ---------------------------------------------------------------------------
