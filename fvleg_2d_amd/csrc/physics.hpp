@@ -132,12 +132,13 @@ __device__ inline Prim<double> cons_to_prim(double r, double ru, double rv, doub
   return Prim<double>{r, u, v, p};
 }
 
-// 1/x in FP64 to about 1 ulp: hardware estimate plus one third-order step (the
+// 1/x in FP64 to about 1 ulp: hardware estimate plus two Newton steps (the
 // precision form's epilogue; the FP64 form divides).
 __device__ inline double rcp64(double x) {
-  const double r = __builtin_amdgcn_rcp(x);
+  double r = __builtin_amdgcn_rcp(x);
   double e = __builtin_fma(-x, r, 1.0);
-  e = __builtin_fma(e, e, e);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-x, r, 1.0);
   return __builtin_fma(r, e, r);
 }
 
@@ -161,10 +162,9 @@ __device__ inline Prim<double> cons_to_prim_fast(double r, double ru, double rv,
 // the quotient with one correction (v_div_fmas) and a special-case fix-up
 // (v_div_fixup); sqrt(x) to an input scaling below 2^-767, v_rsq, Goldschmidt
 // steps, the inverse scaling and a select for 0 / inf.  While the scalings are
-// identities and no special case arises, what is left without those steps gives
-// the same bits: a quotient corrected once from a rounded reciprocal is the
-// rounded quotient.  FastOps is that remainder, with the reciprocal of a shared
-// denominator formed once.  The
+// identities and no special case arises, dropping those steps leaves the same
+// operations on the same values, hence the same bits.  FastOps is that
+// remainder, with the reciprocal of a shared denominator formed once.  The
 // stage kernel uses it only on tiles whose operands keep every division in
 // range (numerator 0 or |a| >= 2^-969, 2^-1021 <= |b| < 2^1021, normal
 // quotient, exponents less than 768 apart; square roots of 2^-767 <= x < inf)
@@ -184,15 +184,19 @@ struct IeeeOps {
 };
 struct FastOps {
   template <typename T> struct Rcp { double b, y; };
-  // v_rcp_f64 is within 2^-24.3 (measured over a binade), so one third-order step,
-  // y (1 + e + e^2) with e = 1 - b y exact to 2^-77, is within 2^-72 before its last
-  // rounding: the rounded reciprocal except where that lies within 2^-19 ulp of a
-  // tie, in three operations where two Newton steps take four.
+  // Two Newton steps, as in the division.  One third-order step, y (1 + e + e^2),
+  // would save an operation (3 % of 1024^2 cells with HLLC + MLP5: 39.0 ms a pass of 128
+  // steps, 40.2 so) but not the bits: it is within 2^-73 of 1 / b before its last
+  // rounding, and where 1 / b lies closer than that to a tie (some 400 of 2^35 random b,
+  // 3,000 of the 2^33 largest ones below 2) y can be the wrong neighbour.  A third of
+  // those near 2 have a numerator whose quotient then rounds the wrong way.
   static __device__ Rcp<double> rcp(double b) {
-    const double y = __builtin_amdgcn_rcp(b);
+    double y = __builtin_amdgcn_rcp(b);
     double e = __builtin_fma(-b, y, 1.0);
-    e = __builtin_fma(e, e, e);
-    return Rcp<double>{b, __builtin_fma(y, e, y)};
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    return Rcp<double>{b, y};
   }
   // y = 1 / b formed once, correctly rounded
   static __device__ Rcp<double> rcp_of(double b, double y) { return Rcp<double>{b, y}; }

@@ -43,3 +43,50 @@ def test_zero_rates_keep_their_sign(oracle, flux, nodes, tile):
             assert all((w == 0.0).all() and np.signbit(w).all() for w in want)
         for g, w in zip(got, want):
             assert same_bits(g, w)
+
+
+def next_to_ties(b, count=4):
+    """53-bit numerators whose quotients by the odd b lie next to the middle of two doubles."""
+    out = []
+    for k in (53, 54):  # quotients above and below 1
+        inv = pow(1 << k, -1, b)
+        for r in range(1, 2 * count, 2):
+            out += [a for a in ((r * inv) % b, (-r * inv) % b) if a >= 1 << 52]
+            out += [a + b for a in ((r * inv) % b, (-r * inv) % b) if a + b < 1 << 53]
+    return [a for a in out if a + 1 < 1 << 53]
+
+
+# denominators whose reciprocal, formed in too few steps, is the wrong neighbour of a tie, with numerators whose
+# quotient that reciprocal then rounds the wrong way; and denominators over the binade
+HARD = {0x1FFFFFF4AFB0DD: [0x183AE850BC9D36], 0x1FFFFFF4AFB0D5: [0x1D5DEB16A5FF7B],
+        0x1FFFFFF4AFB0D3: [0x1535056D46796C], 0x1FFFFFF4AFB0D1: [0x19011D77ED891A],
+        0x1FFFFFE95F61A9: [0x12AC9245C236D8], 0x1FFFFFE95F61A3: [0x1B5CC4B3FB7470],
+        0x1FFFFFCEAF47DF: [0x1278331DCFC0B9], 0x1FFFFFCAEF1B07: [0x127C54DE819F71],
+        0x1FFFFFC64FA9AD: [0x14053B8C4F89D1], 0x1FFFFFD66E47C1: [0x1620CE4E284F57]}
+SPREAD = [int(b) | 1 for b in np.random.default_rng(8).integers(1 << 52, 1 << 53, 12)]
+
+
+def two_columns(b1, b2, nj):
+    """Nodes of two columns of cells, b1 2^-52 and b2 2^-52 wide, nj cells of height 1 (and ghost cells)."""
+    def nodes(ni, rows, nh):
+        x = np.concatenate([-b1 * 2.0 ** -52 - np.arange(2 * nh, 0, -2), [-b1 * 2.0 ** -52, 0.0, b2 * 2.0 ** -52],
+                            b2 * 2.0 ** -52 + np.arange(2, 2 * nh + 1, 2)])
+        g = np.meshgrid(x, np.arange(-nh, nj + nh + 1, dtype=np.float64), indexing="ij")
+        return [np.asfortranarray(c) for c in g]
+    return nodes
+
+
+@pytest.mark.parametrize("tile", [-1, 0])
+def test_quotients_of_fluxes_next_to_ties(oracle, tile):
+    """The flux balance divides by the larger flux: pressures b and 2 a - b beside each other make the fluxes b and a,
+    exactly.  (Not with the b of fewer than 2^5 ulp below 2, where the compiler's own division, whose operations these
+    are, rounds some quotients the wrong way.)"""
+    pairs = [(n, b) for b in list(HARD) + SPREAD for n in HARD.get(b, []) + next_to_ties(b) if n < b]
+    a, b = (np.array(c, dtype=np.float64) * 2.0 ** -52 for c in zip(*pairs))
+    p = np.asfortranarray(np.stack([b, 2.0 * a - b]))
+    one, zero = np.ones(p.shape), np.zeros(p.shape)
+    got, want = interior_rates(oracle, [one, zero, zero, p], two_columns(1 << 52, 1 << 52, len(pairs)), "AUSM+", "minmod",
+                               tile=tile)
+    assert np.array_equal(want[1][0], -((a / b - 1.0) * b))
+    for g, w in zip(got, want):
+        assert same_bits(g, w)
