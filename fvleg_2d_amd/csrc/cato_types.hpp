@@ -117,8 +117,8 @@ struct StageArgs {
   const double *dyj, *lyj;   // per halo'd j
   // Uniform rectilinear grid (every interior cell alike): the cell geometry the stage epilogue
   // derives from dxi..lyj, computed once on the host with the same operations: dx, dy, the
-  // bottom / right / top / left edge lengths after their equalisation, the volume and, when
-  // the volume is a power of two (ugeom_pow2), its exact reciprocal.  ugeom = 0: per cell
+  // bottom / right / top / left edge lengths after their equalisation, the volume and its
+  // reciprocal, exact for a power of two (ugeom_pow2), else volume_rcp.  ugeom = 0: per cell
   int ugeom, ugeom_pow2;
   double ug[8];
   const LoopState *loop;     // dt source and done flag (may be null -> dt_value)

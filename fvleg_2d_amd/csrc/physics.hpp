@@ -1077,11 +1077,15 @@ __device__ inline void scaled_pair(double a, double b, double m, double &qa, dou
 
 // d / vol for a cell volume (positive) within [2^-400, 2^400] whose reciprocal the
 // cell's four variables share; |d| over 2^600, inf and NaN, and other volumes take the
-// IEEE division.  A nonzero d is above 2^-101: divergence() flushes each of its two
-// balances below 1e-14 > 2^-47, so that their sum is 0 or at least 2^-53 of one.  The
-// remainder is formed with the opposite sign, and taken back so, because d = -fl is -0
-// wherever nothing flows: q = -0 then stays -0, as in the IEEE division, where the
-// other sign's +0 remainder turns it into +0.
+// IEEE division.  The reciprocal is a rounded quotient of its own, so that one
+// correction gives the rounded quotient of every d; two Newton steps, as in the
+// compiler's division, leave a few reciprocals of volumes within 2^5 ulp below a power
+// of two unrounded, and with them some quotients off by an ulp.  A nonzero d is above
+// 2^-101: divergence() flushes each of its two balances below 1e-14 > 2^-47, so that
+// their sum is 0 or at least 2^-53 of one.  The remainder is formed with the opposite
+// sign, and taken back so, because d = -fl is -0 wherever nothing flows: q = -0 then
+// stays -0, as in the IEEE division, where the other sign's +0 remainder turns it
+// into +0.
 __device__ inline double over_volume(double d, const FastOps::Rcp<double> &vol) {
   if (vol.y != 0.0 && absd(d) <= 0x1p600) {
     const double q = d * vol.y;
@@ -1090,8 +1094,9 @@ __device__ inline double over_volume(double d, const FastOps::Rcp<double> &vol) 
   }
   return d / vol.b;
 }
-__device__ inline FastOps::Rcp<double> volume_rcp(double vol) {
-  return FastOps::Rcp<double>{vol, (vol >= 0x1p-400 && vol <= 0x1p400) ? FastOps::rcp(vol).y : 0.0};
+// That reciprocal, 0 for a volume out of the range (formed on the host for uniform grids).
+__host__ __device__ inline double volume_rcp(double vol) {
+  return (vol >= 0x1p-400 && vol <= 0x1p400) ? 1.0 / vol : 0.0;
 }
 
 // ---------------------------------------------------------------------------

@@ -141,8 +141,8 @@ static int build_quad_geometry(int ni, int nj, int nh, const double *nx, const d
 // The stage epilogue's cell geometry (stage_kernel.hpp, phase 3) when every
 // interior cell has the same dxi, lxi, dyj and lyj, in the kernel's operations
 // (IEEE double on both sides, so the same bits): edge-length equalisation
-// (quad_cell.f90:110-112) over (l1, l2, l1, l2), volume dx dy, and the exact
-// reciprocal of a power-of-two volume.
+// (quad_cell.f90:110-112) over (l1, l2, l1, l2), volume dx dy, and its reciprocal
+// (exact for a power of two, else volume_rcp).
 static void uniform_cell_geometry(int ni, int nj, int nh, Geometry1D &g) {
   g.uniform = false;
   for (int a = nh; a < nh + ni; ++a)
@@ -161,7 +161,7 @@ static void uniform_cell_geometry(int ni, int nj, int nh, Geometry1D &g) {
   const uint64_t ib = (vb & 0x8000000000000000ull) | ((2046 - ve) << 52);
   double inv;
   std::memcpy(&inv, &ib, 8);
-  const double u[8] = {dx, dy, lb, lr, lt, ll, vol, pow2 ? inv : 0.0};
+  const double u[8] = {dx, dy, lb, lr, lt, ll, vol, pow2 ? inv : volume_rcp(vol)};
   for (int k = 0; k < 8; ++k) g.u[k] = u[k];
   g.u_pow2 = pow2;
   g.uniform = true;

@@ -544,8 +544,8 @@ __device__ inline bool load_tile(Args &a, int i0, int j0, Sp &sp, int &err) {
 }
 
 // Geometry of one cell as the epilogue takes it: widths, edge lengths (bottom,
-// right, top, left), volume and its reciprocal (FP64: the exact one of a power of
-// two, else 0; precision form: rounded).
+// right, top, left), volume with the reciprocal of over_volume (FP64, no power of two)
+// and inv_vol: FP64, the exact reciprocal of a power of two; precision form, a rounded one.
 struct CellGeo {
   double dxv, dyv, lb, lr, lt, ll;
   FastOps::Rcp<double> vol;
@@ -597,7 +597,8 @@ template <bool kExact, bool GEOM, class Args> __device__ inline CellGeo cell_geo
     const double inv_pow2 = __longlong_as_double((long long)((vb & 0x8000000000000000ull) | ((2046 - ve) << 52)));
     inv_vol = kExact ? (pow2 ? inv_pow2 : 0.0) : rcp64(vol);
   }
-  const FastOps::Rcp<double> rv = kExact && !pow2 ? volume_rcp(vol) : FastOps::Rcp<double>{vol, 0.0};
+  FastOps::Rcp<double> rv{vol, 0.0};
+  if (kExact && !pow2) rv.y = !GEOM && a.ugeom ? inv_vol : volume_rcp(vol);
   return CellGeo{dxv, dyv, lb, lr, lt, ll, rv, inv_vol, pow2};
 }
 

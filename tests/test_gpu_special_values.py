@@ -90,3 +90,20 @@ def test_quotients_of_fluxes_next_to_ties(oracle, tile):
     assert np.array_equal(want[1][0], -((a / b - 1.0) * b))
     for g, w in zip(got, want):
         assert same_bits(g, w)
+
+
+@pytest.mark.parametrize("tile", [-1, 0])
+def test_quotients_by_the_volume_next_to_ties(oracle, tile):
+    """d / volume in two columns of cells: a pressure jump of a 2^-53 between them makes d = a 2^-54, exactly."""
+    widths = list(HARD) + SPREAD + [(1 << 53) - k for k in (1, 3, 5)]
+    for b1, b2 in zip(widths, widths[1:] + widths[:1]):
+        a = [n for b in (b1, b2) for n in HARD.get(b, []) + next_to_ties(b)]
+        nj = len(a)
+        lo = np.full(nj, 2.0 ** -53)
+        p = np.asfortranarray(np.stack([np.array(a, dtype=np.float64) * 2.0 ** -53 + lo, lo]))
+        one, zero = np.ones((2, nj)), np.zeros((2, nj))
+        got, want = interior_rates(oracle, [one, zero, zero, p], two_columns(b1, b2, nj), "AUSM+", "minmod", tile=tile)
+        d = np.array(a, dtype=np.float64) * 2.0 ** -54
+        assert np.array_equal(want[1], np.stack([d / (b1 * 2.0 ** -52), d / (b2 * 2.0 ** -52)]))
+        for g, w in zip(got, want):
+            assert same_bits(g, w)
