@@ -710,12 +710,16 @@ __device__ inline void flux_ausmpw(const Gas<R> &gas, int low_mach_fix, const Ed
 }
 
 // Roe (reference variant): roe_solver.fypp:420-511, f_h 519-527
-template <typename R> __device__ inline R roe_f_h(R pL, R pR) {
+template <typename R, class D = IeeeOps> __device__ inline R roe_f_h(R pL, R pR) {
   const R a = absd(pR - pL), b = fmin2(pR, pL) + R(1e-16);
-  // FP64: the rounded quotient a / b is below 1 exactly where a < b or b < 0
-  // (a >= 0; neighbouring binary64 numbers differ by at least 2^-53 relative, so
-  // no a < b rounds up to 1; NaN and infinite operands compare alike)
-  if constexpr (std::is_same<R, double>::value) return (a < b || b < R(0)) ? R(0) : R(1);
+  // FP64: the rounded quotient a / b is below 1 exactly where a < b (a >= 0;
+  // neighbouring binary64 numbers differ by at least 2^-53 relative, so no a < b
+  // rounds up to 1) or where b is negative and a / b a number: a is no NaN (b may
+  // still be one of the two pressures) and b finite (where it is -inf, a is inf).
+  // On FastOps tiles the pressures are positive and finite.
+  if constexpr (std::is_same<D, FastOps>::value) return (a < b) ? R(0) : R(1);
+  if constexpr (std::is_same<R, double>::value)
+    return (a < b || (b < R(0) && a >= R(0) && b >= R(-1.7976931348623157e308))) ? R(0) : R(1);
   const R ratio = a / b;
   return (ratio < R(1)) ? R(0) : R(1);
 }
@@ -779,17 +783,17 @@ __device__ inline void flux_roe(const Gas<R> &gas, const EdgeState<R> &s, const 
   // f_p (roe_solver.fypp:496-507); f_h is symmetric in its two pressures.
   R fp;
   if (edge_ax0<R, DIR>(s)) {
-    fp = roe_f_h(pn.p00, pn.p10);            // (i,j)   (i+1,j)
-    fp = fmax2(fp, roe_f_h(pn.p00, pn.p0p)); // (i,j)   (i,j+1)
-    fp = fmax2(fp, roe_f_h(pn.p00, pn.p0m)); // (i,j)   (i,j-1)
-    fp = fmax2(fp, roe_f_h(pn.p0p, pn.p1p)); // (i,j+1) (i+1,j+1)
-    fp = fmax2(fp, roe_f_h(pn.p0m, pn.p1m)); // (i,j-1) (i+1,j-1)
+    fp = roe_f_h<R, D>(pn.p00, pn.p10);            // (i,j)   (i+1,j)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p00, pn.p0p)); // (i,j)   (i,j+1)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p00, pn.p0m)); // (i,j)   (i,j-1)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p0p, pn.p1p)); // (i,j+1) (i+1,j+1)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p0m, pn.p1m)); // (i,j-1) (i+1,j-1)
   } else {
-    fp = roe_f_h(pn.p00, pn.p10);            // (i,j)   (i,j+1)
-    fp = fmax2(fp, roe_f_h(pn.p00, pn.p0m)); // (i,j)   (i-1,j)
-    fp = fmax2(fp, roe_f_h(pn.p00, pn.p0p)); // (i,j)   (i+1,j)
-    fp = fmax2(fp, roe_f_h(pn.p10, pn.p1m)); // (i,j+1) (i-1,j+1)
-    fp = fmax2(fp, roe_f_h(pn.p10, pn.p1p)); // (i,j+1) (i+1,j+1)
+    fp = roe_f_h<R, D>(pn.p00, pn.p10);            // (i,j)   (i,j+1)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p00, pn.p0m)); // (i,j)   (i-1,j)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p00, pn.p0p)); // (i,j)   (i+1,j)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p10, pn.p1m)); // (i,j+1) (i-1,j+1)
+    fp = fmax2(fp, roe_f_h<R, D>(pn.p10, pn.p1p)); // (i,j+1) (i+1,j+1)
   }
   out[1] = out[1] - R(0.5) * fp * rav * cav * (-(du_trans * ny) + psi * du * nx);
   out[2] = out[2] - R(0.5) * fp * rav * cav * (du_trans * nx + psi * du * ny);

@@ -107,3 +107,23 @@ def test_quotients_by_the_volume_next_to_ties(oracle, tile):
         assert np.array_equal(want[1], np.stack([d / (b1 * 2.0 ** -52), d / (b2 * 2.0 ** -52)]))
         for g, w in zip(got, want):
             assert same_bits(g, w)
+
+
+# Roe's sensor next to pressures that are not a number or minus infinity: neighbours whose other terms are all 0
+@pytest.mark.parametrize("odd", [np.nan, -np.inf, np.inf, -2.0])
+def test_sensor_of_odd_pressures(oracle, odd):
+    cfg = SchemeConfig(flux="Roe", limiter="minmod", bcs=OPEN)
+    ni, nj, nh = 21, 18, cfg.n_ghost
+    x, y = uniform_nodes(ni, nj, nh)
+    ocfg = oracle.Config(ni, nj, flux="Roe", limiter="minmod", bcs=OPEN)
+    rng = np.random.default_rng(7)
+    p = np.full((ni + 2 * nh, nj + 2 * nh), -1.0, order="F")
+    p[nh::4, nh::4] = odd
+    edges = [np.asfortranarray(rng.uniform(0.3, 1.5, (2, ni + 1, nj + 1))) for _ in range(8)]
+    one = np.ones_like(p)
+    with np.errstate(all="ignore"):
+        want = oracle.edge_fluxes(ocfg, oracle.Geometry(ocfg, x, y), one, one, one, p, edges)
+        with Solver(cfg, x, y) as s:
+            got = s.edge_fluxes(edges, p)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
