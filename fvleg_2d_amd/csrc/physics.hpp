@@ -831,14 +831,17 @@ __device__ inline void flux_ausm_plus(const Gas<R> &gas, const EdgeState<R> &s, 
   R M_half = M_sum + R(0);
   if (absd(M_half) < R(1e-13)) M_half = R(0);
   // supersonic: half (M + |M|) over M, which FP64 writes without the division: 1 or 0
-  // (NaN for an infinite M; the sign of a zero is lost in the sum below)
+  // (the sign of a zero is lost in the sum below), but for an M whose double is
+  // infinite, 2^1022 and above being left to the division (FastOps: |M| < 2^170)
   auto super_plus = [](R M) {
-    if constexpr (std::is_same<R, double>::value) return (M > R(0) ? R(1) : R(0)) + (M - M);
-    else return (R(0.5) * (M + absd(M))) / M;
+    if constexpr (std::is_same<R, double>::value)
+      if (std::is_same<D, FastOps>::value || absd(M) <= R(0x1p1022)) return M > R(0) ? R(1) : R(0);
+    return (R(0.5) * (M + absd(M))) / M;
   };
   auto super_minus = [](R M) {
-    if constexpr (std::is_same<R, double>::value) return (M < R(0) ? R(1) : R(0)) + (M - M);
-    else return (R(0.5) * (M - absd(M))) / M;
+    if constexpr (std::is_same<R, double>::value)
+      if (std::is_same<D, FastOps>::value || absd(M) <= R(0x1p1022)) return M < R(0) ? R(1) : R(0);
+    return (R(0.5) * (M - absd(M))) / M;
   };
   R P_plus = (absd(M_L) >= R(1)) ? super_plus(M_L)
                                   : M2p_L * ((R(2) - M_L) - R(16) * alpha * M_L * M2m_L);

@@ -127,3 +127,34 @@ def test_sensor_of_odd_pressures(oracle, odd):
             got = s.edge_fluxes(edges, p)
     for g, w in zip(got, want):
         assert np.array_equal(g, w)
+
+
+# AUSM+ where twice a finite Mach number is infinite: half of that over the Mach number is infinite, not 1, and
+# times a zero normal not a number
+def test_mach_numbers_near_the_largest_double(oracle):
+    cfg = SchemeConfig(flux="AUSM+", limiter="minmod", bcs=OPEN)
+    ni, nj, nh = 5, 4, cfg.n_ghost
+    x, y = uniform_nodes(ni, nj, nh)
+    ocfg = oracle.Config(ni, nj, flux="AUSM+", limiter="minmod", bcs=OPEN)
+    shape = (2, ni + 1, nj + 1)
+    # [0]: the left, [1]: the right state of an edge; a sound speed near 2e-162 beside speeds that make Mach numbers
+    # on both sides of 2^1022 and 2^1023
+    speed = np.array([1.0, 9.0, 11.0, 19.0, 21.0, 29.0])[:, None] * 1e145 * np.ones((1, nj + 1))
+    for side, sign in ((0, 1.0), (1, -1.0)):
+        e = [np.ones(shape, order="F") for _ in range(8)]
+        for k in (2, 3, 4, 5):
+            e[k][:] = 0.0
+        for k in (2, 5):  # u on the i-edges, v on the j-edges
+            e[k][side] = sign * speed
+        for k in (3, 4):  # the other component, so that no mass flux meets a zero speed
+            e[k][side] = 1.0
+        for k in (6, 7):
+            e[k][1 - side] = 5e-324
+        one = np.ones((ni + 2 * nh, nj + 2 * nh), order="F")
+        with np.errstate(all="ignore"):
+            want = oracle.edge_fluxes(ocfg, oracle.Geometry(ocfg, x, y), one, one, one, one, e)
+            with Solver(cfg, x, y) as s:
+                got = s.edge_fluxes(e, one)
+        assert np.isinf(want[0]).any() and np.isnan(want[0]).any()
+        for g, w in zip(got, want):
+            assert np.array_equal(g, w, equal_nan=True)
