@@ -590,6 +590,26 @@ static __global__ void k_pack_ghosts(FieldGeom g, int ld, size_t n, const double
   ghosts[(size_t)blockIdx.y * m + k] = fields[blockIdx.y * n + ghost_cell(k, g.ni, g.nj, g.nh, ld)];
 }
 
+// The interior of four halo'd fields (rows of ld, n elements each) into a pitched set
+// (fs elements a field), and back between zeros, whole rows.
+static __global__ void k_from_halo(FieldGeom g, int ld, size_t n, const double *__restrict__ halo, size_t fs,
+                                   double *__restrict__ set) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= g.ni) return;
+  for (int j = blockIdx.y; j < g.nj; j += gridDim.y)
+    set[blockIdx.z * fs + (size_t)j * g.pitch + i] = halo[blockIdx.z * n + (size_t)(j + g.nh) * ld + (i + g.nh)];
+}
+static __global__ void k_to_halo(FieldGeom g, int ld, size_t n, const double *__restrict__ set, size_t fs,
+                                 double *__restrict__ halo) {
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x, i = ii - g.nh;
+  if (ii >= ld) return;
+  for (int jj = blockIdx.y; jj < g.nj + 2 * g.nh; jj += gridDim.y) {
+    const int j = jj - g.nh;
+    const bool in = i >= 0 && i < g.ni && j >= 0 && j < g.nj;
+    halo[blockIdx.z * n + (size_t)jj * ld + ii] = in ? set[blockIdx.z * fs + (size_t)j * g.pitch + i] : 0.0;
+  }
+}
+
 // muscl_interpolation_t%interpolate_edge_values on a halo'd field q:
 // edges (2, 0:ni, 0:nj) for both directions.
 template <typename R, int LIMC>

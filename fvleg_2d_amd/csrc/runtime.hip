@@ -719,8 +719,8 @@ struct cato_ctx {
   // arguments change (energy source, diagnostics)
   hipGraphExec_t steps_exec = nullptr;
   bool use_graph = true;
-  // operator calls on the caller's halo'd fields: device memory for them and pinned host memory for the
-  // ghost cells they return, of the largest call so far, freed with the context
+  // operator calls on the caller's halo'd fields: device memory for those that do not fit the free primitive
+  // sets (OpMemory) and pinned host memory for the ghost cells they return, both freed with the context
   double *op_mem = nullptr, *op_host = nullptr;
   size_t op_elems = 0, op_host_elems = 0;
 };
@@ -862,7 +862,6 @@ namespace {
 int launch_pressure_column(cato_ctx *c, const StageArgs &a, const PressureInput &pa) {
   Solve &s = c->s;
   FieldGeom g = s.fgeom();
-  g.pitch = a.pitch;
   double *d[4];
   for (int v = 0; v < 4; ++v) d[v] = const_cast<double *>(a.prim[v]);
   const bool recover = s.cfg.precision != CATO_PRECISION_FP64 && a.mode != MODE_RESIDUAL;
@@ -1568,16 +1567,44 @@ int cato_get_timing(cato_ctx *c, double *stage_ms, long long *stage_n, double *o
 }
 
 // ---- operator-level entry points -------------------------------------------
-// Device memory for n doubles of an operator call.
-static int op_workspace(cato_ctx *c, size_t n) {
-  if (n <= c->op_elems) return CATO_OK;
-  if (c->op_mem) (void)hipFree(c->op_mem);
-  c->op_mem = nullptr;
-  c->op_elems = 0;
-  int rc = hip_check(hipMalloc((void **)&c->op_mem, n * sizeof(double)), "operator workspace");
-  if (!rc) c->op_elems = n;
-  return rc;
-}
+// Device memory of one operator call for n doubles.  Between calls two of a context's three primitive sets are
+// free.  They lie side by side unless a subcycled step has swapped one of them with the current set, and then hold
+// 8 fields: the boundary fill, the flux solver and the reconstruction take 4 to 5, a little larger for their halos,
+// so only narrow grids (less than about 2 n_ghost cells across) and rows much wider than the grid need memory of
+// their own.  That is kept for the next call up to kOpKeep; what exceeds it (the 25 to 41 fields of the edge fluxes)
+// is given back when the call ends, so that a context holds no more of the device than its solve.
+constexpr size_t kOpKeep = ((size_t)64 << 20) / sizeof(double);
+struct OpMemory {
+  cato_ctx *c;
+  double *p = nullptr;
+  explicit OpMemory(cato_ctx *ctx) : c(ctx) {}
+  OpMemory(const OpMemory &) = delete;
+  OpMemory &operator=(const OpMemory &) = delete;
+  ~OpMemory() {
+    if (c->op_elems > kOpKeep) release();
+  }
+  void release() {
+    if (c->op_mem) (void)hipFree(c->op_mem);
+    c->op_mem = nullptr;
+    c->op_elems = 0;
+  }
+  int take(size_t n) {
+    double *const lo = std::min(c->s.P[1][0], c->s.P[2][0]), *const hi = std::max(c->s.P[1][0], c->s.P[2][0]);
+    const size_t set = 4 * c->s.field_elems();
+    if (hi == lo + set && n <= 2 * set) {
+      p = lo;
+      return CATO_OK;
+    }
+    if (n > c->op_elems) {
+      release();
+      int rc = hip_check(hipMalloc((void **)&c->op_mem, n * sizeof(double)), "operator workspace");
+      if (rc) return rc;
+      c->op_elems = n;
+    }
+    p = c->op_mem;
+    return CATO_OK;
+  }
+};
 
 // The caller's halo'd primitives (rows of ld, n elements each) into D and their ghost cells filled there;
 // launched, not waited for.  The ghosts come back packed, through return_ghosts after the stream's work.
@@ -1624,7 +1651,8 @@ int cato_apply_bc(cato_ctx *c, double *rho, double *u, double *v, double *p, int
   if (ld < s.ni + 2 * s.nh) return fail(CATO_ERR_INVALID, "ld < ni + 2*nh");
   const size_t n = (size_t)ld * (s.nj + 2 * s.nh);
   double *H[4] = {rho, u, v, p};
-  if ((rc = op_workspace(c, 4 * n)) || (rc = fill_ghosts(c, H, ld, n, c->op_mem))) return rc;
+  OpMemory mem(c);
+  if ((rc = mem.take(4 * n)) || (rc = fill_ghosts(c, H, ld, n, mem.p))) return rc;
   HIPCK(hipStreamSynchronize(c->stream));
   return_ghosts(c, H, ld);
   return CATO_OK;
@@ -1638,8 +1666,9 @@ int cato_interpolate_edges(cato_ctx *c, const double *q, int ld, double *i_edges
   int nx = s.ni + 2 * s.nh, ny = s.nj + 2 * s.nh;
   if (ld < nx) return fail(CATO_ERR_INVALID, "ld < ni + 2*nh");
   size_t n = (size_t)ld * ny, ne = (size_t)2 * (s.ni + 1) * (s.nj + 1);
-  if ((rc = op_workspace(c, n + 2 * ne))) return rc;
-  double *Q = c->op_mem, *IE = Q + n, *JE = IE + ne;
+  OpMemory mem(c);
+  if ((rc = mem.take(n + 2 * ne))) return rc;
+  double *Q = mem.p, *IE = Q + n, *JE = IE + ne;
   HIPCK(hipMemcpyAsync(Q, q, n * 8, hipMemcpyHostToDevice, c->stream));
   FieldGeom g = s.fgeom();
   dim3 grid((unsigned)((ne + 255) / 256));  // 2 * (ni+1)*(nj+1) threads
@@ -1666,8 +1695,9 @@ int cato_edge_fluxes(cato_ctx *c, const double *edges, const double *p, int ld, 
   size_t n = (size_t)ld * ny, ne = (size_t)2 * (s.ni + 1) * (s.nj + 1);
   size_t nfi = (size_t)4 * (s.ni + 1) * s.nj, nfj = (size_t)4 * s.ni * (s.nj + 1);
   const size_t nedge = (s.cfg.flux == FLUX_M_AUSMPW_PLUS ? 16 : 8) * ne;  // + superbee states
-  if ((rc = op_workspace(c, nedge + n + nfi + nfj))) return rc;
-  double *E = c->op_mem, *P = E + nedge, *FI = P + n, *FJ = FI + nfi;
+  OpMemory mem(c);
+  if ((rc = mem.take(nedge + n + nfi + nfj))) return rc;
+  double *E = mem.p, *P = E + nedge, *FI = P + n, *FJ = FI + nfi;
   HIPCK(hipMemcpyAsync(E, edges, nedge * 8, hipMemcpyHostToDevice, c->stream));
   HIPCK(hipMemcpyAsync(P, p, n * 8, hipMemcpyHostToDevice, c->stream));
   FieldGeom g = s.fgeom();
@@ -1702,22 +1732,23 @@ int cato_residual(cato_ctx *c, double *rho, double *u, double *v, double *p, dou
   if (!rho || !u || !v || !p) return fail(CATO_ERR_INVALID, "null field pointer");
   if (ld < s.ni + 2 * s.nh) return fail(CATO_ERR_INVALID, "ld < ni + 2*nh");
   // 1. boundary fill of the caller's halo'd primitives (intent(inout) in the reference)
-  const size_t n = (size_t)ld * (s.nj + 2 * s.nh), inner = (size_t)s.nh + (size_t)s.nh * ld;
+  const size_t n = (size_t)ld * (s.nj + 2 * s.nh), f = s.field_elems();
   double *H[4] = {rho, u, v, p};
-  if ((rc = op_workspace(c, 8 * n)) || (rc = fill_ghosts(c, H, ld, n, c->op_mem))) return rc;
-  // 2. residual from the interior of the same fields (ghosts resolved in-kernel by the same BC map, the +x
-  //    outflow and pressure input by their ghost column), written between zeroed halos.  The stage kernel
-  //    takes the caller's rows as they are: copied row by row into the pitched state buffers and back they
-  //    cost 3,872 copies and 33 ms of a 640 x 481 call whose kernels take 32 us
-  double *D0 = c->op_mem, *O = D0 + 4 * n;
-  HIPCK(hipMemsetAsync(O, 0, 4 * n * sizeof(double), c->stream));
+  OpMemory mem(c);
+  if ((rc = mem.take(4 * n)) || (rc = fill_ghosts(c, H, ld, n, mem.p))) return rc;
+  // 2. residual from the interior primitives (ghosts resolved in-kernel by the same BC map); scratch: the two state
+  //    buffers that do not hold U^n, so a pending initial state survives.  Repacked on the device: the caller's
+  //    rows copied one by one into the pitched buffers and back were 3,872 copies and 33 ms of a 640 x 481 call
+  //    whose kernels take 32 us (1.2 ms so)
+  double **Pbuf = s.U[(s.cur + 1) % 3], **Obuf = s.U[(s.cur + 2) % 3];
+  FieldGeom g = s.fgeom();
+  const unsigned rows = (unsigned)std::min(s.nj + 2 * s.nh, 32768);
+  hipLaunchKernelGGL(k_from_halo, dim3((unsigned)((s.ni + 255) / 256), rows, 4), dim3(256), 0, c->stream, g, ld, n,
+                     (const double *)mem.p, f, Pbuf[0]);
+  HIPCK(hipGetLastError());
+  if ((rc = fill_outflow_column(c->stream, s, Pbuf))) return rc;
   StageArgs a = s.stage_args(MODE_RESIDUAL, 0, 0, 0, -1, -1, (s.cur + 2) % 3, 0, -1, false, nullptr, 1.0, false);
-  for (int k = 0; k < 4; ++k) {
-    a.prim[k] = D0 + k * n + inner;
-    a.out[k] = O + k * n + inner;
-  }
-  a.pitch = ld;
-  a.fstride = (long long)n;
+  for (int k = 0; k < 4; ++k) a.prim[k] = Pbuf[k];
   a.block_min = nullptr;
   a.block_err = nullptr;
   if ((rc = validate_stage_args(a))) return rc;
@@ -1727,7 +1758,11 @@ int cato_residual(cato_ctx *c, double *rho, double *u, double *v, double *p, dou
   dim3 grid((unsigned)(s.tiles_x * s.tiles_y));
   s.launcher(grid, c->stream, a);
   HIPCK(hipGetLastError());
-  for (int k = 0; k < 4; ++k) HIPCK(hipMemcpyAsync(D[k], O + k * n, n * 8, hipMemcpyDeviceToHost, c->stream));
+  // the rates between zeroed halos, over the primitives they came from
+  hipLaunchKernelGGL(k_to_halo, dim3((unsigned)((ld + 255) / 256), rows, 4), dim3(256), 0, c->stream, g, ld, n,
+                     (const double *)Obuf[0], f, mem.p);
+  HIPCK(hipGetLastError());
+  for (int k = 0; k < 4; ++k) HIPCK(hipMemcpyAsync(D[k], mem.p + k * n, n * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCK(hipStreamSynchronize(c->stream));
   return_ghosts(c, H, ld);
   return CATO_OK;
