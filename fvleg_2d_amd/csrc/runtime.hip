@@ -1762,10 +1762,10 @@ int cato_residual(cato_ctx *c, double *rho, double *u, double *v, double *p, dou
   hipLaunchKernelGGL(k_to_halo, dim3((unsigned)((ld + 255) / 256), rows, 4), dim3(256), 0, c->stream, g, ld, n,
                      (const double *)Obuf[0], f, mem.p);
   HIPCK(hipGetLastError());
-  for (int k = 0; k < 4; ++k) HIPCK(hipMemcpyAsync(D[k], mem.p + k * n, n * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCK(hipStreamSynchronize(c->stream));
-  return_ghosts(c, H, ld);
-  return CATO_OK;
+  return_ghosts(c, H, ld);  // before the rates, which may go into the same arrays
+  for (int k = 0; k < 4; ++k) HIPCK(hipMemcpyAsync(D[k], mem.p + k * n, n * 8, hipMemcpyDeviceToHost, c->stream));
+  return hip_check(hipStreamSynchronize(c->stream), "residual");
 }
 
 }  // extern "C"

@@ -79,3 +79,15 @@ def test_residual_after_subcycled_steps():
     for a, b in zip(got[:half], got[half:]):
         for x, y in zip(a, b):
             assert np.array_equal(x, y)
+
+
+def test_rates_in_the_primitives_own_arrays():
+    """Every value of a rate array is the rate (0 in the halo), also where it is one of the primitives' arrays."""
+    cfg = SchemeConfig(flux="SLAU", limiter="minmod", bcs=("zero_gradient",) * 4)
+    with Solver(cfg, *uniform_nodes(33, 25, cfg.n_ghost)) as s:
+        halo = halo_fields(s, cfg.n_ghost)
+        want = s.residual(*[a.copy(order="F") for a in halo])
+        ptr = [a.ctypes.data_as(DP) for a in halo]
+        N.check(s.lib.cato_residual(s.h, *ptr, *ptr, s.halo_shape()[0]), "residual")
+        for x, y in zip(halo, want):
+            assert np.array_equal(x, y)
