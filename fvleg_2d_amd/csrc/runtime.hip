@@ -325,24 +325,24 @@ int Solve::init(const cato_config &c, const cato_geom &g, bool single) {
 
 size_t Solve::field_elems() const { return (size_t)pitch * nj; }
 
-// Tiles whose partials device_bytes() counts: the solve's own, or where the library chose them the 32 x 8
-// ones (quad cells: 16 x 16) that every single solve once had, so that a footprint does not depend on the
-// choice.  A single solve's partials lie in its tail.
+// Tiles whose partials device_bytes() counts: those of an explicit tile, else the 32 x 8 ones of the server
+// (quad cells, which have no served form: 16 x 16), so that a footprint does not depend on the library's choice.
 size_t Solve::counted_tiles() const {
   const TileShape t = kTiles[cfg.tile >= 0 && !geo.quad ? tile : geo.quad ? kQuadTile : 0];
   return (size_t)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty);
 }
 
-size_t Solve::device_bytes() const {
+size_t Solve::core_bytes() const {
   size_t f = field_elems();
-  size_t nb = counted_tiles();
   size_t geo_n = (size_t)2 * (ni + 2 * nh) + 2 * (nj + 2 * nh);
   return (12 + 12) * f * sizeof(double) + geo_n * sizeof(double) + (size_t)Q_COUNT * quad_elems() * sizeof(double) +
-         nb * (sizeof(double) + sizeof(int)) + sizeof(LoopState) + 4 * sizeof(double) + 1024;
+         sizeof(LoopState) + 4 * sizeof(double) + 1024;
 }
 
-// Carve the device arrays of one solve out of `base` (device_bytes() long).
-void Solve::bind(char *base) {
+size_t Solve::device_bytes() const { return core_bytes() + counted_tiles() * (sizeof(double) + sizeof(int)); }
+
+// Carve the device arrays of one solve out of `base` (device_bytes() long; core_bytes() without the partials).
+void Solve::bind(char *base, bool partials) {
   size_t f = field_elems();
   double *p = reinterpret_cast<double *>(base);
   for (int s = 0; s < 3; ++s)
@@ -361,16 +361,19 @@ void Solve::bind(char *base) {
   lyj = p; p += nj + 2 * nh;
   quad = geo.quad ? p : nullptr;
   p += (size_t)Q_COUNT * quad_elems();
-  block_min = p; p += counted_tiles();
+  if (partials) {
+    block_min = p;
+    p += counted_tiles();
+  }
   result = p; p += 4;
   char *c = reinterpret_cast<char *>(p);
   c = reinterpret_cast<char *>(((uintptr_t)c + 255) & ~(uintptr_t)255);
   loop = reinterpret_cast<LoopState *>(c);
   c += sizeof(LoopState);
-  block_err = reinterpret_cast<int *>(c);
+  if (partials) block_err = reinterpret_cast<int *>(c);
 }
 
-// What a single solve keeps after its device_bytes(): the second copies of the loop state and the sanity
+// What a single solve keeps after its core_bytes(): the second copies of the loop state and the sanity
 // flags (StageArgs::fold_n), and the partials of its tiles.
 size_t Solve::tail_bytes() const {
   return 256 + sizeof(LoopState) + (size_t)tiles_x * tiles_y * (sizeof(double) + 2 * sizeof(int));
@@ -1016,14 +1019,14 @@ int cato_ctx_create(const cato_config *cfg, const cato_geom *geom, cato_ctx **ou
     delete c;
     return rc;
   }
-  size_t bytes = c->s.device_bytes();
-  if ((rc = hip_check(hipMalloc(&c->mem, bytes + c->s.tail_bytes()), "device allocation"))) {
+  const size_t core = c->s.core_bytes();
+  if ((rc = hip_check(hipMalloc(&c->mem, core + c->s.tail_bytes()), "device allocation"))) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     return rc;
   }
-  c->s.bind(c->mem);
-  c->s.bind_tail(c->mem + bytes);
+  c->s.bind(c->mem, false);
+  c->s.bind_tail(c->mem + core);
   if ((rc = c->s.upload_geometry(c->stream)) || (rc = hip_check(hipStreamSynchronize(c->stream), "sync"))) {
     cato_ctx_destroy(c);
     return rc;

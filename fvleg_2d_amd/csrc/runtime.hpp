@@ -72,8 +72,9 @@ struct Solve {
   size_t quad_elems() const { return geo.quad ? (size_t)(ni + 2 * nh) * (nj + 2 * nh) : 0; }
   size_t field_elems() const;
   size_t counted_tiles() const;
+  size_t core_bytes() const;
   size_t device_bytes() const;
-  void bind(char *base);
+  void bind(char *base, bool partials = true);
   size_t tail_bytes() const;
   void bind_tail(char *base);
   int upload_geometry(hipStream_t s);

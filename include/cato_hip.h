@@ -283,8 +283,13 @@ int cato_batch_set_pressure_input(cato_batch *b, int k, const double *time, cons
 int cato_batch_run(cato_batch *b, const double *max_time, const double *contour_interval_dt, long long max_iterations,
                    int use_graph, long long *iterations, double *times, int *errors);
 
-/* Device memory one solve of this configuration and grid occupies (its HBM
- * footprint, as the serving form charges it against its budget).  Needs no
+/* Device memory one solve of this configuration and grid occupies in the
+ * serving form (what a server charges against its budget).  A context of its
+ * own takes the same but for its loop state's second copy and the partials of
+ * its own tile (12 to 16 bytes a tile), and what its caller asks for beside:
+ * an energy source, a pressure table, diagnostics, and up to 64 MiB that
+ * operator calls keep when their fields do not fit what the context has free
+ * (rows much wider than the grid, a few cells across, edge fluxes).  Needs no
  * device. */
 int cato_device_bytes(const cato_config *cfg, const cato_geom *geom, unsigned long long *bytes);
 
