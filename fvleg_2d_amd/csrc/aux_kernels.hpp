@@ -204,12 +204,12 @@ static __global__ __launch_bounds__(1024) void k_close_step(int nb, const double
   close_step<1024, 8>(nb, block_min, block_err, out, L, mode);
 }
 
-// k_close_step with the convergence norms of the step (cv.sums): the block sums of
-// squares are added in a fixed order (threads, then waves), so the norms are the
-// same on every run; NORM2's own order agrees to a few ulps.
-static __global__ __launch_bounds__(1024) void k_reduce_finalize(int nb, double *__restrict__ block_min,
-                                                          int *__restrict__ block_err, double *__restrict__ out,
-                                                          LoopState *__restrict__ L, int mode, ConvOut cv) {
+// k_close_step with the convergence norms of the step, in one pass over the partials:
+// the block sums of squares are added in a fixed order (threads, then waves), so the
+// norms are the same on every run; NORM2's own order agrees to a few ulps.
+static __global__ __launch_bounds__(1024) void k_close_step_norms(int nb, const double *__restrict__ block_min,
+                                                           int *__restrict__ block_err, double *__restrict__ out,
+                                                           LoopState *__restrict__ L, int mode, ConvOut cv) {
   __shared__ double sm[16];
   __shared__ int se[16];
   __shared__ double ss[16][8];
@@ -217,57 +217,41 @@ static __global__ __launch_bounds__(1024) void k_reduce_finalize(int nb, double 
   // One workgroup reads every partial: the loop is latency-bound, so each
   // thread issues kU partials (and their 8 convergence sums) before using any.
   constexpr int kU = 4;
-  const bool conv = cv.sums != nullptr;
   double m = __builtin_inf();
   int e = 0;
   double t[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) t[v] = 0.0;
   for (int b0 = threadIdx.x; b0 < nb; b0 += kU * blockDim.x) {
-    double x[kU];
+    double x[kU], c[kU][8];
     int f[kU];
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
       const int b = b0 + k * (int)blockDim.x;
       x[k] = b < nb ? block_min[b] : __builtin_inf();
       f[k] = b < nb ? block_err[b] : 0;
-    }
-    if (conv) {
-      double c[kU][8];
 #pragma unroll
-      for (int k = 0; k < kU; ++k) {
-        const int b = b0 + k * (int)blockDim.x;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) c[k][v] = b < nb ? cv.sums[(size_t)v * nb + b] : 0.0;
-      }
-#pragma unroll
-      for (int k = 0; k < kU; ++k)
-#pragma unroll
-        for (int v = 0; v < 8; ++v) t[v] = t[v] + c[k][v];
+      for (int v = 0; v < 8; ++v) c[k][v] = b < nb ? cv.sums[(size_t)v * nb + b] : 0.0;
     }
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
-      const int b = b0 + k * (int)blockDim.x;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) t[v] = t[v] + c[k][v];
       m = (x[k] < m) ? x[k] : m;
       e |= f[k];
-      if (b < nb && f[k]) block_err[b] = 0;
+      if (f[k]) block_err[b0 + k * (int)blockDim.x] = 0;
     }
   }
   m = wave_min(m);
   e = wave_or(e);
   const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) / 64;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) t[v] = wave_sum(t[v]);
   if ((threadIdx.x & 63) == 0) {
     sm[w] = m;
     se[w] = e;
-  }
-  if (conv) {
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      double y = t[v];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) y = y + __shfl_xor(y, o, 64);
-      if ((threadIdx.x & 63) == 0) ss[w][v] = y;
-    }
+    for (int v = 0; v < 8; ++v) ss[w][v] = t[v];
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
@@ -275,35 +259,29 @@ static __global__ __launch_bounds__(1024) void k_reduce_finalize(int nb, double 
     m = (sm[k] < m) ? sm[k] : m;
     e |= se[k];
   }
-  double nrm[4] = {0.0, 0.0, 0.0, 0.0};
-  if (conv) {
-    double sum[8];
-    for (int v = 0; v < 8; ++v) {
-      sum[v] = ss[0][v];
-      for (int k = 1; k < nw; ++k) sum[v] = sum[v] + ss[k][v];
-    }
-    // norm2(last - first) / norm2(first); the momenta divide by max(norm2(first), 1)
-    for (int v = 0; v < 4; ++v) {
-      double den = sqrt(sum[4 + v]);
-      if (v == 1 || v == 2) den = den > 1.0 ? den : 1.0;
-      nrm[v] = sqrt(sum[v]) / den;
-      cv.norms[v] = nrm[v];
-    }
+  double nrm[4], sum[8];
+  for (int v = 0; v < 8; ++v) {
+    sum[v] = ss[0][v];
+    for (int k = 1; k < nw; ++k) sum[v] = sum[v] + ss[k][v];
   }
-  if (out) {
-    out[0] = m;
-    out[1] = (double)e;
+  // norm2(last - first) / norm2(first); the momenta divide by max(norm2(first), 1)
+  for (int v = 0; v < 4; ++v) {
+    double den = sqrt(sum[4 + v]);
+    if (v == 1 || v == 2) den = den > 1.0 ? den : 1.0;
+    nrm[v] = sqrt(sum[v]) / den;
+    cv.norms[v] = nrm[v];
   }
-  const double step_dt = (mode == 2) ? L->dt : 0.0;
+  out[0] = m;
+  out[1] = (double)e;
+  if (mode != 2) return;
+  const double step_dt = L->dt;
   loop_update(L, m, e, mode);
-  if (mode == 2 && conv && cv.hist) {
-    // write_residual_history (mod_fluid.f90:1207-1223) row of the step just closed
-    double *row = cv.hist + (size_t)((L->iteration - 1) % cv.hist_cap) * kHistRow;
-    row[0] = (double)L->iteration;
-    row[1] = L->master_time;
-    row[2] = step_dt;
-    for (int v = 0; v < 4; ++v) row[3 + v] = nrm[v];
-  }
+  // write_residual_history (mod_fluid.f90:1207-1223) row of the step just closed
+  double *row = cv.hist + (size_t)((L->iteration - 1) % cv.hist_cap) * kHistRow;
+  row[0] = (double)L->iteration;
+  row[1] = L->master_time;
+  row[2] = step_dt;
+  for (int v = 0; v < 4; ++v) row[3 + v] = nrm[v];
 }
 
 static __global__ void k_set_scalar(double *dst, double value) { *dst = value; }

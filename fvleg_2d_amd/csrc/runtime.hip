@@ -910,8 +910,8 @@ int launch_reduce(cato_ctx *c, int mode, bool with_conv) {
     // the convergence sums belong to a step (modes 0 and 2 after stages), not to a CFL pass
     const ConvOut cv = with_conv ? s.conv_out() : ConvOut{};
     if (cv.sums)
-      hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(1024), 0, c->stream, nb, s.block_min, s.block_err, s.result,
-                         s.loop, mode, cv);
+      hipLaunchKernelGGL(k_close_step_norms, dim3(1), dim3(1024), 0, c->stream, nb, (const double *)s.block_min,
+                         s.block_err, s.result, s.loop, mode, cv);
     else
       hipLaunchKernelGGL(k_close_step, dim3(1), dim3(1024), 0, c->stream, nb, (const double *)s.block_min, s.block_err,
                          s.result, s.loop, mode);
