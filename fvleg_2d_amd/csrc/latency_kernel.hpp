@@ -153,8 +153,8 @@ __global__ __launch_bounds__(4 * TX * TY) void latency_kernel(StageArgs a) {
   const bool in_range = load_tile<FLUX, LIMC, R, TX, TY, NT, false>(a, i0, j0, sm.sp, err);
   // The FastOps flux of the SLAU family and HLLC only: AUSM+, AUSMPW+ and Roe divide
   // as IEEE does here.  Their FastOps forms shorten no chain (Sod 400 x 4 with AUSM+ 2 %
-  // slower) and take Roe to 159 registers, three workgroups a CU instead of five
-  // (301 x 243, rk(2,4), superbee: 6.39 -> 6.65 ms).
+  // slower) and take Roe from 115 to 159 registers, three workgroups a CU instead of
+  // four (301 x 243, rk(2,4), superbee, in this layout: 6.39 -> 6.65 ms a pass).
   constexpr bool kFastFlux = slau_family<FLUX>() || FLUX == FLUX_HLLC;
   constexpr bool kFastScheme = kExact && (kFastFlux || LIMC == LIM_MLP3 || LIMC == LIM_MLP5);
   if constexpr (kFastScheme) {

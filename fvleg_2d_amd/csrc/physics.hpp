@@ -1048,7 +1048,8 @@ __device__ inline void edge_flux(const Gas<R> &gas, int low_mach_fix, const Edge
 // FP64 fluxes with a FastOps path (every one but M-AUSMPW+; every limiter has
 // one), and the bound B of fast_ops_cell that keeps a scheme's operations in
 // range: 60 for TVD2 with the SLAU family, 20 otherwise.  What it took off a stage
-// of 1024 x 987 cells on 32 x 8 tiles, van Leer / MLP5 (the range vote included):
+// of 1024 x 987 cells on 32 x 8 tiles, van Leer / MLP5 (the range vote included, the
+// reciprocals an operation shorter than they are now):
 // AUSM+ 73.5 -> 67.0 / 119.6 -> 109.7 us, AUSMPW+ 88.0 -> 77.8 / 134.7 -> 121.8 us,
 // Roe 93.7 -> 80.0 / 139.0 -> 122.2 us.
 template <int FLUX> constexpr bool slau_family() {
@@ -1068,8 +1069,9 @@ template <int FLUX> constexpr bool needs_pressure_nbrs() {
 // or |b| itself, and x / |x| is exactly copysign(1, x), so one division gives both
 // quotients bit for bit.  Below 2^1000 it is the FastOps one: the other operand is
 // at most m, and where it is so small (below 2^-969) that the quotient's correction
-// loses bits, the quotient is lost beside the 1 anyway.  Larger m, inf and NaN keep
-// both IEEE divisions.
+// loses bits, what they change, 2^-1021 of a length, is lost beside the 1 or, where the
+// larger flux's edge has no length, below the balance's flush (1e-14 m), for lengths up
+// to 2^900.  Larger m, inf and NaN keep both IEEE divisions.
 __device__ inline void scaled_pair(double a, double b, double m, double &qa, double &qb) {
   if (!(m <= 0x1p1000)) {
     qa = a / m;

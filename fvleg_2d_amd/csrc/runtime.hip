@@ -254,26 +254,40 @@ static int validate_config(const cato_config &c) {
   return CATO_OK;
 }
 
-// The library's choice of tile for a solve with launches of its own.
+// The library's choice of tile for a solve with launches of its own.  Figures: us per SSP-RK3 step of square grids,
+// the end-of-step reduction included, each group of tiles timed in turns on one box.
 //
-// Up to five 8 x 8 tiles per CU: the latency layout.  Measured with five schemes in both precisions, us per
-// SSP-RK3 step with 32 x 8 tiles / in the latency layout: 64^2 35-51 / 21-25 (FP64) and 26-35 / 15-17 (FP32
-// flux); 256^2 35-52 / 32-43 and 25-35 / 21-27; 272^2 (1156 tiles) 40-64 / 36-49 and 28-40 / 23-30; FP64
-// 288^2 (1296 tiles) 40-64 / 42-58.  Four per CU in FP64 with TVD2 under the SLAU family, Roe and M-AUSMPW+: more
-// than 96 registers leave a CU four of their workgroups, and a second round costs more than it saves.  16 x 16
-// tiles / latency layout at 254^2 (1024 tiles) and 270^2 (1156): Roe + superbee 36.1 / 37.7 and 43.6 / 47.9 us,
-// SLAU2 + minmod 32.8 / 32.2 and 38.4 / 41.4, SD-SLAU + superbee 34.5 / 34.1 and 41.5 / 44.0, M-AUSMPW+ + minmod
-// 44.1 / 43.9 and 52.2 / 54.7; where it stays (MLP, the other fluxes), SLAU2 + MLP3 50.4 / 47.0, Roe + MLP5
-// 62.4 / 57.3, HLLC + minmod 39.3 / 37.1.
+// Up to five 8 x 8 tiles per CU: the latency layout.  16 x 16 tiles (32 x 8 ones are within 2 %, MLP5 5 % slower) /
+// latency layout, FP64 and FP32 flux:
+//   64^2  SLAU + van Leer 33 / 21 and 24 / 15, HLLC + MLP5 47 / 25 and 31 / 17
+//   270^2 (1156 tiles)  HLLC + minmod 41.2 / 39.8 and 27.4 / 24.7, SLAU2 + MLP3 51.7 / 48.4 and 33.3 / 28.5,
+//         Roe + MLP5 64.6 / 59.1 and 39.2 / 34.3
+//   286^2 (1296 tiles, a sixth round of workgroups on some CUs)  HLLC + minmod 41.1 / 46.3 and 27.9 / 26.7,
+//         SLAU2 + MLP3 51.6 / 52.9 and 33.5 / 31.1, Roe + MLP5 64.3 / 65.4 and 39.4 / 37.8
+// Four per CU in FP64 with TVD2 under the SLAU family, Roe and M-AUSMPW+: their 101 to 117 registers leave a CU four
+// of the 256-thread workgroups (96 and fewer leave five), and a second round costs more than it saves.
+//   254^2 (1024 tiles)  Roe + superbee 38.7 / 39.4, SLAU2 + minmod 35.4 / 34.4, SD-SLAU + superbee 37.1 / 36.4,
+//         M-AUSMPW+ + minmod 47.1 / 45.7
+//   262^2 (1089 tiles)  44.3 / 47.6, 38.8 / 42.5, 41.9 / 45.3, 53.6 / 55.4
+// MLP makes a tile dear enough for five there too (270^2 above).
 //
-// Above, 32 x 16 where its fewer edges and halo cells per cell pay: with at least four such tiles per CU (with
-// fewer, the last round of tiles is too empty: 640^2, 3.1 per CU, is 3 to 8 % slower), in FP64 unless the
-// scheme's registers take its occupancy (Roe, AUSMPW+ and M-AUSMPW+ with MLP5: 2 to 4 % slower), and in the
-// precision form with MLP5 or from 1.5 M cells on.  Elsewhere 16 x 16.  us a stage with 16 x 16 / 32 x 16
-// tiles (32 x 8): FP64 1024^2 HLLC + MLP5 108.4 / 103.9 (111.7), Roe + superbee 73.7 / 76.9 (76.2), 2048^2 Roe +
-// superbee 257.8 / 269.1 (253.2), SLAU + van Leer 231.7 / 228.5 (231.0), AUSMPW+ + MLP5 (older kernels) 421 / 434
-// (424); FP32 flux 1024^2 HLLC + MLP5 55.0 / 54.2 (57.4), SLAU + van Leer 34.3 / 34.5 (34.6), 2048^2 125.2 / 119.2
-// (125.9).
+// Above, 32 x 16 where its fewer edges and halo cells per cell pay: with at least four such tiles per CU, in FP64
+// unless the scheme's registers take its occupancy, in the precision form with MLP5 or from 1.5 M cells on.  Elsewhere
+// 16 x 16.  16 x 16 / 32 x 16 (32 x 8):
+//   FP64  640^2 (3.1 tiles per CU: the last round is too empty)  SLAU + van Leer 89 / 97 (90), HLLC + MLP5 147 / 153
+//         (148), Roe + superbee 98 / 108 (98)
+//   1024^2  HLLC + MLP5 299 / 290 (303), SLAU + van Leer 173 / 172 (175), Roe + superbee 188 / 204 (193)
+//   2048^2  HLLC + MLP5 1132 / 1108 (1157), SLAU + van Leer 654 / 643 (652), Roe + superbee 699 / 725 (715)
+//   AUSMPW+, M-AUSMPW+ and Roe with MLP5 were 2 to 4 % slower on 32 x 16 when this line was drawn; AUSMPW+ has
+//   fewer divisions since and, like M-AUSMPW+, is left 1 to 2 % behind on 16 x 16: 1024^2 323 / 321 and 369 / 364,
+//   2048^2 1206 / 1197 and 1382 / 1359; Roe 320 / 316 and 1204 / 1189
+//   FP32 flux  1024^2 (1.05 M)  HLLC + MLP5 150 / 148 (158), SLAU + van Leer 91.7 / 93.0 (92.9), HLLC + minmod
+//         89.7 / 93.3 (90.7), SLAU2 + MLP3 124.0 / 123.9 (128.7)
+//   1260^2 (1.59 M)  224 / 220 (226), 130 / 131 (131), 126 / 130 (128), 182 / 181 (183)
+//   1400^2 (1.96 M)  270 / 265 (272), 155 / 155 (155), 152 / 153 (151), 220 / 215 (221)
+//   1600^2 (2.56 M)  342 / 326 (345), 193 / 187 (197), 187 / 183 (190), 274 / 261 (276)
+//   2048^2 (4.19 M)  533 / 516 (539), 321 / 307 (317), 313 / 301 (306), 433 / 405 (428)
+// kCus: the library is built for gfx950 alone, which has 256.
 constexpr int kCus = 256;
 constexpr int kLatencyTiles = 5 * kCus;
 
