@@ -733,8 +733,9 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
   // ---- 1. primitives of the tile + halo ---------------------------------
   // A wave that loads its tile issues before waves of other workgroups that are at
   // their edges: its few instructions start a wait of microseconds that those
-  // waves' arithmetic then covers (KH 2048^2 FP64 245 -> 236 us, Riemann 1024^2 HLLC +
-  // MLP5 104 -> 99 us, precision form 1 %; the other way round it was 1 % slower).
+  // waves' arithmetic then covers (Riemann 1024^2 HLLC + MLP5 97.6 -> 92.3 us a stage,
+  // precision form 0.5 %, KH 2048^2 FP64 the same now that the epilogue's loads are asked
+  // for ahead, 4 % before; the other way round it was 1 % slower).
   // The precision form and MLP ask for all their cells at once: one memory latency
   // for the tile instead of one per round of the workgroup over its cells (1 to 2 %
   // of a stage; FP64 TVD2 is 2 % slower so, and the batched kernel spills).
@@ -767,10 +768,11 @@ __device__ inline void stage_tile(Args &a, int tile, double dt, TileSmem<LIMC, R
   // What a thread's cell reads from memory (its states, the geometry of a
   // quadrilateral cell) is asked for before the barrier: one latency, under the wait
   // for the slowest wave, where the epilogue's branches (mode, division fallbacks) had
-  // made it one per variable, one after the other.  Stages: KH 2048^2 FP64 206 -> 203 us,
-  // precision form 111 -> 102 us; Riemann 1024^2 HLLC + MLP5 91 -> 89 us; quadrilateral
-  // 500 x 421 25.0 -> 23.5 us.  Asking before the edge pass (registers held through it)
-  // and for the edge normals ahead gave nothing more.
+  // made it one per variable, one after the other.  Stages when this was taken: KH 2048^2
+  // FP64 206 -> 203 us, precision form 111 -> 102 us; Riemann 1024^2 HLLC + MLP5 91 -> 89 us;
+  // quadrilateral 500 x 421 25.0 -> 23.5 us.  Nearly all of it is asking for all of them
+  // together: after the barrier they cost the same within 1 %.  Asking before the edge pass
+  // (registers held through it) and for the edge normals ahead gave nothing more.
   constexpr bool kOneCell = NT == TX * TY;
   CellInputs own;
   CellGeo own_geo;
